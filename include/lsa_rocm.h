@@ -227,6 +227,22 @@ int lsa_read(const void* q, const void* k, const void* v, int dtype, int64_t B, 
              const int32_t* ids, const int32_t* lengths, int32_t W, int ids_per_head, float scale, int empty_nan,
              int32_t splits, int32_t* counters, void* scratch, size_t scratch_bytes, void* out, void* stream);
 
+/* The same read for many query rows over one cache (the reference's prefill: every row has
+ * its own list), as a masked sweep on the matrix cores: 256 query columns (rows times the
+ * kv-head's query group) a workgroup cross the 64-key tiles any of their rows lists, each
+ * row's list a bitmap that masks its weights (16-bit halves that add up to the fp32 weight
+ * within 2^-17). Rows the sweep does not serve - a list naming a key twice, a tile whose K or V
+ * is not finite, too few listed keys for the tiles crossed - are read by the gather in the
+ * same call. Arguments as lsa_read's; bf16/fp16 rows of head dim 64 or 128, at most 262144
+ * cache rows, kv_token_stride below 2^24, scale > 0. lsa_read_rows_scratch_bytes(): 0 where it
+ * does not apply; scratch 256-byte aligned, no initialisation. */
+size_t lsa_read_rows_scratch_bytes(int dtype, int64_t B, int64_t Tq, int64_t Tk, int32_t Hq, int32_t Hkv, int32_t D,
+                                   int32_t W, int ids_per_head);
+int lsa_read_rows(const void* q, const void* k, const void* v, int dtype, int64_t B, int64_t Tq, int64_t Tk,
+                  int32_t Hq, int32_t Hkv, int32_t D, int64_t kv_batch_stride, int64_t kv_token_stride,
+                  int64_t kv_head_stride, const int32_t* ids, const int32_t* lengths, int32_t W, int ids_per_head,
+                  float scale, int empty_nan, void* scratch, size_t scratch_bytes, void* out, void* stream);
+
 /* Chunked prefill read: query row t of chunk c = t / chunk reads chunk c's per-kv-head
  * list ids [B, C, Hkv, W] (first lengths[b, c, g] slots) plus the chunk's causal block
  * [c*chunk, t]. q [B, T, Hq, D], k/v [B, Tk, Hkv, D], out like q; T <= Tk.

@@ -1,0 +1,828 @@
+// The per-row sparse read as a masked sweep on the matrix cores, for many query rows (the
+// reference's prefill: every row has its own list, read_kernel_tiled.py:30-156).
+//
+// The gather read fetches each row's list for itself: at 32k rows of 4612 keys that is 576 GB
+// through the L2s (12.5 TB/s, 46 ms) for a cache of 134 MB. Rows that are neighbours list much
+// of the same cache, so here 256 query columns (32-row blocks times the kv-head's query group)
+// sweep the 64-key tiles any of their rows lists, and each row's list, as a bitmap over the
+// cache rows, masks the softmax weights: the keys outside it weigh exactly zero.
+//
+//   tile_finite_kernel  flags the 64-key tiles whose K or V holds a value that is not finite
+//                       (a masked product would not be zero there);
+//   row_bits_kernel     turns 32 rows' lists into bitmaps (bits [block][tile][row], 64 bits
+//                       each) and flags, per block and tile, whether any row lists a key there,
+//                       and the rows that list a key twice (a bitmap cannot count);
+//   rows_mfma_kernel    the sweep, 256 columns a workgroup;
+//   rows_rest_kernel    the gather read of the rows the sweep leaves out: a duplicate in the
+//                       list, a flagged tile among the workgroup's, or too few listed keys for
+//                       the tiles they are spread over.
+//
+// A slab of query rows at a time, so that the bitmaps stay under kSlabBytes.
+#include <math.h>
+
+#include "lsa_abi_common.h"
+#include "lsa_mfma_dev.h"
+#include "lsa_read_dev.h"
+
+using namespace lsa;
+
+namespace {
+
+constexpr int kTile = 64;              // keys of a tile
+constexpr int kWaves = 8;
+constexpr int kThreads = 64 * kWaves;
+constexpr int NB = 4;                  // K and V tile buffers each
+constexpr int kBlockRows = 32;         // query rows of a bitmap block (and columns of a wave)
+constexpr int kMaxTiles = 4096;        // tiles of a cache (262144 rows)
+constexpr int64_t kSlabBytes = 64 << 20;
+constexpr float kGrow = 8.0f;          // log2 growth of a column maximum that forces a rescale
+
+struct RowsArgs {
+  const void* q;
+  const void* k;
+  const void* v;
+  void* out;
+  const int32_t* ids;
+  const int32_t* lengths;
+  int64_t Tq, Tk;
+  int64_t kv_sb, kv_st, kv_sh;
+  int Hq, Hkv, W;
+  int per_head;        // lists per (row, kv-head); 0: one list a row, shared by the heads
+  int64_t u0;          // first row tile of the slab (row tile u = batch * n_rt + tile)
+  int n_u;             // row tiles of the slab
+  int n_rt;            // row tiles a batch row
+  int rb;              // 32-row blocks of a row tile (8 / query group)
+  int n_tile;          // 64-key tiles of the cache
+  uint64_t* bits;      // [block][tile][32 rows]
+  uint8_t* any;        // [block][tile]
+  uint8_t* dup;        // [block][32 rows]
+  uint8_t* rest;       // [row tile][kv-head]: 1 the sweep leaves the tile to the gather
+  const uint8_t* odd;  // [batch of K][kv-head][tile]: a value that is not finite
+  float scale_log2;
+  int empty_nan;
+};
+
+// The list index of query row t of batch b for kv-head g.
+__device__ __forceinline__ int64_t list_of(const RowsArgs& a, int64_t b, int64_t t, int g) {
+  const int64_t row = b * a.Tq + t;
+  return a.per_head ? row * a.Hkv + g : row;
+}
+
+// ---------------------------------------------------------------- tiles that are not finite
+
+template <typename T>
+__device__ __forceinline__ bool odd16(const uint4& x) {  // any of 8 elements infinite or NaN
+  constexpr uint32_t E = __is_same(T, bf16_t) ? 0x7F80u : 0x7C00u;
+  const uint32_t w[4] = {x.x, x.y, x.z, x.w};
+  bool bad = false;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) bad |= (w[i] & E) == E || (w[i] & (E << 16)) == (E << 16);
+  return bad;
+}
+
+// grid (tile, kv-head, batch of K). HBM-bound: one read of K and V.
+template <typename T, int D>
+__global__ __launch_bounds__(LSA_BLOCK) void tile_finite_kernel(RowsArgs a, uint8_t* odd) {
+  constexpr int SEGS = D / 8, N = kTile * SEGS / LSA_BLOCK;
+  __shared__ int bad[LSA_WAVES];
+  const int tile = blockIdx.x, g = blockIdx.y, b = blockIdx.z;
+  const T* kb = (const T*)a.k + b * a.kv_sb + g * a.kv_sh;
+  const T* vb = (const T*)a.v + b * a.kv_sb + g * a.kv_sh;
+  uint4 x[2 * N];
+#pragma unroll
+  for (int n = 0; n < N; ++n) {
+    const int i = n * LSA_BLOCK + threadIdx.x;
+    const int64_t row = min((int64_t)tile * kTile + i / SEGS, a.Tk - 1);
+    const int64_t off = row * a.kv_st + (i % SEGS) * 8;
+    x[2 * n] = *(const uint4*)(kb + off);
+    x[2 * n + 1] = *(const uint4*)(vb + off);
+  }
+  bool o = false;
+#pragma unroll
+  for (int n = 0; n < 2 * N; ++n) o |= odd16<T>(x[n]);
+  const uint64_t m = __ballot(o);
+  if ((threadIdx.x & 63) == 0) bad[threadIdx.x / 64] = m != 0;
+  __syncthreads();
+  if (threadIdx.x == 0)
+    odd[((int64_t)b * gridDim.y + g) * a.n_tile + tile] = (uint8_t)(bad[0] | bad[1] | bad[2] | bad[3]);
+}
+
+// ---------------------------------------------------------------- bitmaps
+
+constexpr int kBitThreads = 1024;
+constexpr int kSegKeys = 32768;                  // cache rows whose bits are in LDS at once
+constexpr int kSegWords = kSegKeys / 32 + 2;     // dwords of a row in LDS (two of padding: conflict-free columns)
+
+struct BitLds {
+  uint32_t w[kBlockRows][kSegWords];
+  int dup[kBlockRows];
+};
+
+// One 32-row block (grid: row tile of the slab, kv-head when lists are per head, block). Two
+// rows a wave; a list is read once per kSegKeys cache rows. LDS-atomic bound.
+__global__ __launch_bounds__(kBitThreads) void row_bits_kernel(RowsArgs a) {
+  __shared__ BitLds sh;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid / 64;
+  const int64_t blk = blockIdx.x;
+  const int rb = (int)(blk % a.rb);
+  const int64_t x = blk / a.rb;
+  const int g = a.per_head ? (int)(x % a.Hkv) : 0;
+  const int64_t u = a.u0 + (a.per_head ? x / a.Hkv : x);
+  const int64_t b = u / a.n_rt;
+  const int64_t t0 = ((u % a.n_rt) * a.rb + rb) * kBlockRows;
+  if (tid < kBlockRows) sh.dup[tid] = 0;
+  for (int64_t k0 = 0; k0 < a.Tk; k0 += kSegKeys) {
+    for (int i = tid; i < kBlockRows * kSegWords; i += kBitThreads) (&sh.w[0][0])[i] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int rr = 0; rr < 2; ++rr) {
+      const int r = 2 * w + rr;
+      const int64_t t = t0 + r;
+      if (t < a.Tq) {
+        const int64_t li = list_of(a, b, t, g);
+        int n = a.lengths[li];
+        n = n < 0 ? 0 : (n > a.W ? a.W : n);
+        const int32_t* list = a.ids + li * a.W;
+        bool twice = false;
+        for (int j0 = 0; j0 < n; j0 += 8 * 64) {
+          int32_t id[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {  // unconditional (clamped): all in flight
+            const int j = j0 + 64 * e + lane;
+            const int32_t v = list[j < n ? j : n - 1];
+            id[e] = j < n ? v : -1;
+          }
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const int64_t o = (int64_t)id[e] - k0;
+            if (id[e] >= 0 && id[e] < a.Tk && o >= 0 && o < kSegKeys) {
+              const uint32_t bit = 1u << (o & 31);
+              twice |= (atomicOr(&sh.w[r][o >> 5], bit) & bit) != 0;
+            }
+          }
+        }
+        if (__any(twice) && lane == 0) sh.dup[r] = 1;
+      }
+    }
+    __syncthreads();
+    const int tiles = (int)min((int64_t)kSegKeys / kTile, (a.Tk - k0 + kTile - 1) / kTile);
+    const int tile0 = (int)(k0 / kTile);
+    for (int i = tid; i < tiles * kBlockRows; i += kBitThreads) {  // 64 lanes: two tiles of 32 rows
+      const int tile = i / kBlockRows, r = i % kBlockRows;
+      const uint64_t word = *(const uint64_t*)&sh.w[r][2 * tile];
+      a.bits[(blk * a.n_tile + tile0 + tile) * kBlockRows + r] = word;
+      const uint64_t m = __ballot(word != 0);
+      if (r == 0) a.any[blk * a.n_tile + tile0 + tile] = (uint8_t)(((lane ? m >> 32 : m) & 0xFFFFFFFFull) != 0);
+    }
+    __syncthreads();
+  }
+  if (tid < kBlockRows) a.dup[blk * kBlockRows + tid] = (uint8_t)sh.dup[tid];
+}
+
+// ---------------------------------------------------------------- the sweep
+//
+// A workgroup is 8 waves of 32 query columns; K and V tiles go from memory straight to LDS
+// (dma16), four buffers each. A wave's step is two phases: M, the last tile's P V products and
+// this tile's scores (matrix cores, LDS reads and the loads ahead), and V, this tile's weights
+// (vector unit). The waves form two groups of four, one wave of each on every SIMD, half a step
+// apart (phase_barrier twice a step), so one group's matrix work runs beside the other's vector
+// work instead of all waves wanting the same unit at once.
+//
+// What bounds it (cycle counts of a wave, D 128): M ~2350 cycles against 1536 of matrix work
+// (issuing the five loads costs ~130 each, wherever they stand), V ~2600 (~330 vector
+// instructions, 32 of them exponentials, beside the other group's matrix instructions). 32k rows
+// of the reference's lists (4288 keys a row on average), Hq 32, Hkv 8, D 128: 10.8 ms against
+// 46.2 for the gather, 1220 TFLOP/s on the products of every swept pair with both halves.
+
+
+template <int D>
+struct alignas(1024) SweepLds {
+  uint16_t k[NB][kTile * D];  // 16-byte segments of a row permuted by kseg
+  uint16_t v[NB][kTile * D];  // by vseg
+  uint64_t mask[kWaves][NB][kBlockRows];
+  uint16_t act[kMaxTiles];    // the tiles swept, ascending
+  int wsum[kWaves], wkeys[kWaves];
+  int bad, n_act;
+};
+
+// Listed keys a swept tile under which the gather reads a workgroup's rows faster: the sweep
+// takes a CU ~2.6 us a tile (D 64: 1.9), the gather ~7.9 ns a listed key (D 64: 2.7, 3.8, 5.9
+// and 12.3 ns at query groups 1, 2, 4 and 8).
+template <int D, int GQ>
+__device__ constexpr int sparse_keys() {
+  return D == 128 ? 330 : (GQ == 1 ? 700 : (GQ == 2 ? 500 : (GQ == 4 ? 320 : 155)));
+}
+
+// Which LDS segment of row r holds its segment 0 (XOR): K rows are read 16 rows to a
+// 16-lane group at one segment, V rows (transposing reads) 8 rows at 64 bytes each.
+template <int D> __device__ __forceinline__ int kseg(int r) { return D == 128 ? r & 15 : (r >> 1) & 7; }
+template <int D> __device__ __forceinline__ int vseg(int r) { return D == 128 ? (r & 3) << 2 : ((r >> 1) & 1) << 2; }
+
+// 1024 (256) bytes from base + voff (a lane's) to LDS address `lds` + 16 (4) * lane, counted
+// by vmcnt. Written as instructions, so that the compiler does not drain the counter before
+// the LDS reads it cannot tell apart from these writes; the waits are wait_vm's.
+__device__ __forceinline__ void dma16(uint32_t lds, const void* base, uint32_t voff) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base)
+               : "memory", "m0");
+}
+__device__ __forceinline__ void dma4(uint32_t lds, const void* base, uint32_t voff) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(voff), "s"(base)
+               : "memory", "m0");
+}
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+__device__ __forceinline__ void phase_barrier() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_barrier" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// What a weight's 16-bit half leaves out, exact in fp32: x - pair.lo (lo) and x - pair.hi (hi),
+// one dot product with (-1, 0) or (0, -1) each. The constants are kept opaque: as an inline
+// operand this compiler gives the packed bf16 pair (-1, 0) the encoding of -1.0, which the
+// instruction reads as the fp32 bits (0, -1).
+template <typename T>
+struct Rest {
+  static constexpr uint32_t ONE = __is_same(T, bf16_t) ? 0xBF80u : 0xBC00u;
+  uint32_t c_lo = ONE, c_hi = ONE << 16;
+  __device__ __forceinline__ Rest() { asm("" : "+s"(c_lo), "+s"(c_hi)); }
+  static __device__ __forceinline__ float dot(uint32_t pair, uint32_t c, float x) {
+    if constexpr (__is_same(T, bf16_t))
+      return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, pair), __builtin_bit_cast(bf16x2_t, c), x, false);
+    else
+      return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2_t, pair), __builtin_bit_cast(f16x2_t, c), x, false);
+  }
+  __device__ __forceinline__ float lo(uint32_t pair, float x) const { return dot(pair, c_lo, x); }
+  __device__ __forceinline__ float hi(uint32_t pair, float x) const { return dot(pair, c_hi, x); }
+};
+
+// All ones where bit `bit` of w is set, else 0 (written as an instruction: with an AND it is two
+// where the compiler's compare and select are three).
+__device__ __forceinline__ uint32_t bit_mask(uint32_t w, int bit) {
+  uint32_t m;
+  asm("v_bfe_i32 %0, %1, %2, 1" : "=v"(m) : "v"(w), "ns"(bit));
+  return m;
+}
+
+// A wave's 32 query columns: LDS addresses, the matrix products, and the weights of a tile. The
+// gather read multiplies fp32 weights, so here a weight enters the matrix cores as the sum of
+// two 16-bit halves, within 2^-17 of it (one half alone would cost 2^-9); the normaliser adds
+// up the fp32 weights.
+template <typename T, int D>
+struct Sweep {
+  using M = Mfma<T>;
+  using op_t = typename M::op_t;
+  static constexpr int KS = D / 16, DB = D / 32, SEGS = D / 8, ROWB = 2 * D;
+  static constexpr int KPI = 1024 / ROWB;            // keys a dma16 moves
+  static constexpr int NI = kTile / (KPI * kWaves);  // dma16s a wave a tile, K and V each
+
+  const lds_char *kl, *vl;
+  uint32_t kbase, vbase;
+  int jj;
+  op_t qop[KS];
+  f32x16_t o[DB], sc[2];
+  uint32_t ph[2][8], pl[2][8];  // the weights' halves, two a word
+  float m_run, l_run;
+  Rest<T> rest;
+
+  __device__ __forceinline__ void init(const void* k_tiles, const void* v_tiles, const T* qrow) {
+    const int lane = threadIdx.x & 63, hh = lane / 32, ln = lane % 32;
+    kl = (const lds_char*)k_tiles;
+    vl = (const lds_char*)v_tiles;
+    jj = (lane % 16) / 4;
+    kbase = (uint32_t)(ln * ROWB) + (uint32_t)((hh ^ kseg<D>(ln)) * 16);  // segment 2 s is this one's XOR 2 s
+    vbase = (uint32_t)((4 * hh + jj) * ROWB + 32 * (ln / 16) + 8 * (lane % 4));
+#pragma unroll
+    for (int s = 0; s < KS; ++s) qop[s] = __builtin_bit_cast(op_t, *(const uint4*)(qrow + 16 * s + 8 * hh));
+#pragma unroll
+    for (int d = 0; d < DB; ++d) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[d][r] = 0.0f;
+    }
+    m_run = kNegBig;
+    l_run = 0.0f;
+  }
+  // Makes the compiler wait for the query rows here, ahead of a loop that counts loads itself.
+  __device__ __forceinline__ void settle_queries() {
+#pragma unroll
+    for (int s = 0; s < KS; ++s) asm volatile("" ::"v"(qop[s]));
+  }
+  // Phase M as groups of matrix operations, each with its LDS operands in a buffer of `op`:
+  // groups 0 .. 3 are O^T += V^T P^T of the last tile (16 keys each), groups 4 .. the scores of
+  // the next (two 16-dim steps each). A group's operands are read while the two groups before
+  // it compute, so the matrix cores do not wait for the LDS.
+  static constexpr int NG = 4 + KS / 2;
+  op_t op[3][4];
+  __device__ __forceinline__ void load_group(int gi, int tile_v, int tile_k) {
+    if (gi < 4) {  // V^T of keys 16 gi .. + 15: dims 32 d + ln at keys {4 hh .. + 3, 8 + 4 hh .. + 3}
+      const lds_char* vt = vl + (tile_v & (NB - 1)) * (kTile * ROWB) + vbase;
+#pragma unroll
+      for (int d = 0; d < DB; ++d) {
+        const lds_char* vd = vt + (uint32_t)(64 * (D == 128 ? (d ^ jj) : (d ^ (jj >> 1))));
+        const uint2 lo = v_column4(vd, 16 * gi * ROWB);
+        const uint2 hi = v_column4(vd, (16 * gi + 8) * ROWB);
+        op[gi % 3][d] = __builtin_bit_cast(op_t, make_uint4(lo.x, lo.y, hi.x, hi.y));
+      }
+    } else if (gi < NG) {  // K rows of both halves at dims 16 s .. + 15, s = 2 (gi - 4) and the next
+      const lds_char* kt = kl + (tile_k & (NB - 1)) * (kTile * ROWB);
+      typedef __attribute__((address_space(3))) const op_t lds_op;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        op[gi % 3][e] = *(lds_op*)(kt + (kbase ^ (uint32_t)(32 * (2 * (gi - 4) + e / 2))) + (e % 2) * 32 * ROWB);
+    }
+  }
+  __device__ __forceinline__ void run_group(int gi) {
+    if (gi < 4) {
+      const int h = gi / 2, sp = gi % 2;
+      const op_t pb = __builtin_bit_cast(op_t, make_uint4(ph[h][4 * sp], ph[h][4 * sp + 1], ph[h][4 * sp + 2], ph[h][4 * sp + 3]));
+#pragma unroll
+      for (int d = 0; d < DB; ++d) o[d] = M::run(op[gi % 3][d], pb, o[d]);
+      const op_t qb = __builtin_bit_cast(op_t, make_uint4(pl[h][4 * sp], pl[h][4 * sp + 1], pl[h][4 * sp + 2], pl[h][4 * sp + 3]));
+#pragma unroll
+      for (int d = 0; d < DB; ++d) o[d] = M::run(op[gi % 3][d], qb, o[d]);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int s = 2 * (gi - 4) + e / 2;
+        sc[e % 2] = M::run(op[gi % 3][e], qop[s], sc[e % 2]);
+      }
+    }
+  }
+  // Tile i's scores, sc[h]: keys 32 h + 8 (r / 4) + 4 hh + r % 4 of column ln (groups 4 .. ;
+  // the first two loaded by load_scores(i)).
+  __device__ __forceinline__ void load_scores(int i) {
+    load_group(4, i, i);
+    load_group(5, i, i);
+  }
+  // hook(g), g = 0, 1, .., is called once a group (loads ahead: the matrix cores stay busy while
+  // they issue).
+  template <typename Hook>
+  __device__ __forceinline__ void run_scores(int i, Hook&& hook) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) sc[h][r] = 0.0f;
+    }
+#pragma unroll
+    for (int gi = 4; gi < NG; ++gi) {
+      load_group(gi + 2, i, i);
+      hook(gi - 4);
+      __builtin_amdgcn_sched_barrier(0);
+      run_group(gi);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  // Tile i's P V product (its first groups loaded by load_pv(i)); loads tile i + 1's scores.
+  __device__ __forceinline__ void load_pv(int i) {
+    __builtin_amdgcn_sched_barrier(0);
+    load_group(0, i, i);
+    load_group(1, i, i);
+  }
+  template <typename Hook>
+  __device__ __forceinline__ void run_pv(int i, Hook&& hook) {
+#pragma unroll
+    for (int gi = 0; gi < 4; ++gi) {
+      load_group(gi + 2, i, i + 1);
+      hook(gi);
+      __builtin_amdgcn_sched_barrier(0);
+      run_group(gi);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+
+  // p = exp2(s * scale - m) of the tile's keys, +0 where the key's bit of wd (this lane's keys of
+  // each half: bit 8 (r / 4) + r % 4) is clear. Eight scores at a time, one operation of all of
+  // them after the other: one wave a SIMD makes weights, so a chain of dependent instructions
+  // would leave the unit idle between them (16k rows: 3.15 ms with four at a time, 2.98 with
+  // eight, 3.00 with sixteen).
+  __device__ __forceinline__ void weights(const uint32_t (&wd)[2], float scale_log2, float (&ls)[2]) {
+    constexpr int E = 8;
+    ls[0] = ls[1] = 0.0f;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int r0 = 0; r0 < 16; r0 += E) {
+        float p[E], q[E];
+        uint32_t m[E];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int e = 0; e < E; ++e) p[e] = fmaf(sc[h][r0 + e], scale_log2, -m_run);
+#pragma unroll
+        for (int e = 0; e < E; ++e) p[e] = fast_exp2(p[e]);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int e = 0; e < E; ++e) m[e] = bit_mask(wd[h], 8 * ((r0 + e) / 4) + e % 4);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int e = 0; e < E; ++e) p[e] = __uint_as_float(__float_as_uint(p[e]) & m[e]);
+        __builtin_amdgcn_sched_barrier(0);
+        uint32_t* pair = &ph[h][r0 / 2];
+#pragma unroll
+        for (int e = 0; e < E; e += 2) pair[e / 2] = M::pack2(p[e], p[e + 1]);
+#pragma unroll
+        for (int e = 0; e < E; ++e) ls[e & 1] += p[e];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int e = 0; e < E; e += 2) {
+          q[e] = rest.lo(pair[e / 2], p[e]);
+          q[e + 1] = rest.hi(pair[e / 2], p[e + 1]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int e = 0; e < E; e += 2) pl[h][(r0 + e) / 2] = M::pack2(q[e], q[e + 1]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  }
+  // The weights of a tile and its share of the normaliser. The running maximum moves lazily:
+  // the weights are made against the current one, and only where a lane's 32 weights reach
+  // 2^kGrow (or are not numbers) are the column maxima taken and, where a column grew by more
+  // than 2^kGrow, the state rescaled and the weights made again. So every weight stays below
+  // 2^kGrow, and most tiles take no maximum.
+  __device__ __forceinline__ void softmax(uint64_t mask, float scale_log2) {
+    const int hh = (threadIdx.x & 63) / 32;
+    const uint32_t wd[2] = {(uint32_t)mask >> (4 * hh), (uint32_t)(mask >> 32) >> (4 * hh)};
+    float ls[2];
+    weights(wd, scale_log2, ls);
+    static_assert(kGrow == 8.0f, "the sum test is against 2^kGrow");
+    if (__any(!(ls[0] + ls[1] < 256.0f))) {
+      float mx = -INFINITY;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, (wd[h] >> (8 * (r / 4) + r % 4)) & 1u ? sc[h][r] : -INFINITY);
+      }
+      const float mt = fmaxf(mx, lane_xor(mx, 32)) * scale_log2;
+      if (__any(mt > m_run + kGrow)) {
+        const float mn = fmaxf(m_run, mt);
+        const float alpha = fast_exp2(m_run - mn);
+        m_run = mn;
+        l_run *= alpha;
+#pragma unroll
+        for (int d = 0; d < DB; ++d) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) o[d][r] *= alpha;
+        }
+        weights(wd, scale_log2, ls);
+      }
+    }
+    l_run += ls[0] + ls[1];
+  }
+  // The normalised output row (lane: 4 dims of every 8 of its column), `empty` where no key weighed.
+  __device__ __forceinline__ void store(T* op, float empty) const {
+    const int hh = (threadIdx.x & 63) / 32;
+    const float lt = l_run + lane_xor(l_run, 32);
+    const float inv = 1.0f / lt;
+    const bool none = !(lt > 0.0f);  // as the gather: a sum that is not a number counts as none
+    if (op == nullptr) return;
+#pragma unroll
+    for (int d = 0; d < DB; ++d) {
+#pragma unroll
+      for (int r4 = 0; r4 < 4; ++r4) {
+        float x[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) x[c] = none ? empty : o[d][4 * r4 + c] * inv;
+        uint2 y;
+        y.x = M::pack2(x[0], x[1]);
+        y.y = M::pack2(x[2], x[3]);
+        *(uint2*)(op + 32 * d + 8 * r4 + 4 * hh) = y;
+      }
+    }
+  }
+};
+
+template <typename T, int D, int GQ>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void rows_mfma_kernel(RowsArgs a) {
+  using S = Sweep<T, D>;
+  constexpr int RB = kWaves / GQ;  // 32-row blocks of the workgroup
+  constexpr int SEGS = S::SEGS, ROWB = S::ROWB, KPI = S::KPI, NI = S::NI;
+  constexpr int PER = 2 * NI + 1;     // loads a wave issues a step
+  constexpr int KLAST = S::NG - 4 - 1;  // the last score group
+  __shared__ SweepLds<D> sh;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int ln = lane % 32;
+  const int g = (int)(blockIdx.x % a.Hkv);
+  const int ul = a.n_u - 1 - (int)(blockIdx.x / a.Hkv);  // later rows list more: longest first
+  const int64_t u = a.u0 + ul;
+  const int64_t b = u / a.n_rt;
+  const int hl = w % GQ, rb = w / GQ;
+  const int64_t t = ((u % a.n_rt) * RB + rb) * kBlockRows + ln;  // this lane's query row
+  const int64_t blk0 = (a.per_head ? (int64_t)ul * a.Hkv + g : ul) * RB;
+  const T* kb = (const T*)a.k + b * a.kv_sb + (int64_t)g * a.kv_sh;
+  const T* vb = (const T*)a.v + b * a.kv_sb + (int64_t)g * a.kv_sh;
+
+  // the tiles any of the workgroup's rows lists, and whether one of them is not finite
+  {
+    if (tid == 0) sh.bad = 0;
+    // the keys its rows list (shared or this kv-head's lists)
+    const int64_t tr = (u % a.n_rt) * RB * kBlockRows + tid;
+    int listed = 0;
+    if (tid < RB * kBlockRows && tr < a.Tq) {
+      const int len = a.lengths[list_of(a, b, tr, g)];
+      listed = len < 0 ? 0 : (len > a.W ? a.W : len);
+    }
+    listed = wave_sum(listed);
+    if (lane == 0) sh.wkeys[w] = listed;
+    __syncthreads();
+    const uint8_t* odd = a.odd + ((a.kv_sb ? b : 0) * a.Hkv + g) * a.n_tile;
+    int base = 0;
+    for (int c0 = 0; c0 < a.n_tile; c0 += kThreads) {
+      const int tile = c0 + tid;
+      const int tc = tile < a.n_tile ? tile : 0;
+      int on = 0;
+#pragma unroll
+      for (int r = 0; r < RB; ++r) on |= a.any[(blk0 + r) * a.n_tile + tc];
+      const bool use = tile < a.n_tile && on;
+      if (use && odd[tc]) sh.bad = 1;
+      const uint64_t m = __ballot(use);
+      if (lane == 0) sh.wsum[w] = __popcll(m);
+      __syncthreads();
+      int before = 0, total = 0;
+#pragma unroll
+      for (int x = 0; x < kWaves; ++x) {
+        before += x < w ? sh.wsum[x] : 0;
+        total += sh.wsum[x];
+      }
+      if (use) sh.act[base + before + __popcll(m & ((1ull << lane) - 1))] = (uint16_t)tile;
+      base += total;
+      __syncthreads();
+    }
+    if (tid == 0) {
+      int keys = 0;
+      for (int x = 0; x < kWaves; ++x) keys += sh.wkeys[x];
+      if (keys < base * sparse_keys<D, GQ>()) sh.bad = 1;
+      sh.n_act = base;
+      a.rest[(int64_t)ul * a.Hkv + g] = (uint8_t)sh.bad;
+    }
+    __syncthreads();
+  }
+  if (sh.bad) return;  // uniform
+  const int n = __builtin_amdgcn_readfirstlane(sh.n_act);
+
+  const bool row_ok = t < a.Tq;
+  const int64_t qrow = ((b * a.Tq + (row_ok ? t : 0)) * a.Hq + (int64_t)g * GQ + hl) * D;
+  S sw;
+  sw.init(&sh.k[0][0], &sh.v[0][0], (const T*)a.q + qrow);
+
+  if (n > 0) {
+    // loads: wave w moves keys [8 w, 8 w + 8) of a K and a V tile, and its own 32 masks
+    const uint32_t st = (uint32_t)a.kv_st * 2u;
+    uint32_t kvo[NI], vvo[NI];
+    auto offsets = [&](int limit) {  // rows at or past `limit` read the row before it
+#pragma unroll
+      for (int x = 0; x < NI; ++x) {
+        const int r = (w * NI + x) * KPI + lane / SEGS;
+        const uint32_t row = (uint32_t)min(r, limit - 1) * st;
+        kvo[x] = row + (uint32_t)(((lane % SEGS) ^ kseg<D>(r)) * 16);
+        vvo[x] = row + (uint32_t)(((lane % SEGS) ^ vseg<D>(r)) * 16);
+      }
+    };
+    const int last_rows = (int)(a.Tk - (int64_t)(a.n_tile - 1) * kTile);  // rows of the cache's last tile
+    const uint32_t k_lds = (uint32_t)(uintptr_t)(lds_char*)&sh.k[0][0];
+    const uint32_t v_lds = (uint32_t)(uintptr_t)(lds_char*)&sh.v[0][0];
+    const uint32_t m_lds = (uint32_t)(uintptr_t)(lds_char*)&sh.mask[w][0][0];
+    const uint64_t* bits = a.bits + (blk0 + rb) * a.n_tile * kBlockRows;
+    // Part x (of NI) of this wave's share of tile i's K or V rows, its i-th tile being `tile`.
+    auto move = [&](uint32_t lds, const T* src, int i, int tile, int x, const uint32_t (&vo)[NI]) {
+      dma16(lds + (uint32_t)(i & (NB - 1)) * (kTile * ROWB) + (uint32_t)(w * NI + x) * 1024u,
+            src + (int64_t)tile * kTile * a.kv_st, vo[x]);
+    };
+    auto load = [&](bool values, int i, int tile, int x) {
+      const bool part = tile == a.n_tile - 1 && last_rows < kTile;  // uniform
+      if (part) offsets(last_rows);
+      if (values) move(v_lds, vb, i, tile, x, vvo);
+      else move(k_lds, kb, i, tile, x, kvo);
+      if (part) offsets(kTile);
+    };
+    auto load_mask = [&](int i, int tile) {
+      dma4(m_lds + (uint32_t)(i & (NB - 1)) * 256u, bits + (int64_t)tile * kBlockRows, (uint32_t)lane * 4u);
+    };
+    auto tile_at = [&](int i) { return __builtin_amdgcn_readfirstlane((int)sh.act[i < n ? i : n - 1]); };
+
+    auto mask_of = [&](int i) {
+      typedef __attribute__((address_space(3))) const uint64_t lds_u8;
+      return *(lds_u8*)((const lds_char*)&sh.mask[w][0][0] + (i & (NB - 1)) * 256 + ln * 8);
+    };
+
+    // Two groups of four waves, one wave of each on every SIMD, half a step apart: while one
+    // group's waves feed the matrix cores (the last tile's P V, this tile's scores), the other
+    // group's make weights. Group 0 runs M(i) in half-step 2 i and V(i) in 2 i + 1, group 1 one
+    // half-step later, so K(i) is read in half-steps 2 i, 2 i + 1 and V(i) in 2 i + 2, 2 i + 3.
+    // In M(i) a wave loads K(i + 3) into the buffer of K(i - 1) (last read in half-step 2 i - 1),
+    // V(i + 2) into that of V(i - 2) (likewise) and its masks of tile i + 3. What a phase reads
+    // was loaded two or more of every wave's M phases before the barrier ahead of it: V(i) is read
+    // from the end of V(i) on (half-step 2 i + 1 at the earliest) and K(i + 1) from half-step
+    // 2 i + 2 on, both loaded in M(i - 2). So at the end of M(i) the loads of M(i) and M(i - 1) may
+    // be outstanding, at the end of V(i) those of M(i).
+    offsets(kTile);
+    int t2 = 0, t3;
+    for (int j = 0; j < 3; ++j) {
+      t2 = tile_at(j);
+#pragma unroll
+      for (int x = 0; x < NI; ++x) {
+        load(false, j, t2, x);
+        if (j < 2) load(true, j, t2, x);
+      }
+      load_mask(j, t2);
+    }
+    t3 = tile_at(3);
+    sw.settle_queries();
+    wait_vm<0>();
+#pragma unroll
+    for (int x = 0; x < NI; ++x) load(false, 3, t3, x);  // M(0)'s
+    phase_barrier();
+    const bool late = w >= kWaves / 2;
+    if (late) phase_barrier();
+    sw.load_scores(0);
+    for (int i = 0;;) {
+      sw.run_scores(i, [&](int x) {
+        if (x < NI) load(true, i + 2, t2, x);
+        if (x == KLAST) load_mask(i + 3, t3);
+      });
+      const uint64_t mask = mask_of(i);
+      wait_vm<2 * PER>();
+      phase_barrier();
+      t2 = t3;
+      t3 = tile_at(i + 4);
+      sw.softmax(mask, a.scale_log2);
+      sw.load_pv(i);
+      wait_vm<PER>();
+      phase_barrier();
+      sw.run_pv(i, [&](int x) {
+        if (x < NI) load(false, i + 4, t3, x);
+      });
+      if (++i == n) break;
+    }
+    if (!late) phase_barrier();
+    wait_vm<0>();  // no load may land after the workgroup's LDS is given back
+  }
+
+  sw.store(row_ok ? (T*)a.out + qrow : nullptr, a.empty_nan ? NAN : 0.0f);
+}
+
+// ---------------------------------------------------------------- the rows left to the gather
+
+// Every workgroup looks at 256 (row, kv-head) units at a time and reads the ones left out.
+template <typename T, int D, int GQ>
+__global__ __launch_bounds__(LSA_BLOCK) void rows_rest_kernel(RowsArgs a) {
+  using S = ReadShape<T, D, GQ>;
+  constexpr int RB = kWaves / GQ, RT = RB * kBlockRows;
+  __shared__ ReadLds<D, GQ, kMaxSplits> sh;
+  __shared__ uint64_t todo[LSA_WAVES];
+  const int tid = threadIdx.x;
+  const int lp = (tid & 63) % S::LPT;
+  const int64_t units = (int64_t)a.n_u * RT * a.Hkv;  // row tile, row, kv-head
+  for (int64_t base = (int64_t)blockIdx.x * LSA_BLOCK; base < units; base += (int64_t)gridDim.x * LSA_BLOCK) {
+    const int64_t i = base + tid;
+    bool left = false;
+    if (i < units) {
+      const int g = (int)(i % a.Hkv);
+      const int64_t x = i / a.Hkv, ul = x / RT;
+      const int r = (int)(x % RT);
+      const int64_t blk = (a.per_head ? ul * a.Hkv + g : ul) * RB + r / kBlockRows;
+      left = a.rest[ul * a.Hkv + g] || a.dup[blk * kBlockRows + r % kBlockRows];
+      left &= ((a.u0 + ul) % a.n_rt) * RT + r < a.Tq;
+    }
+    const uint64_t m = __ballot(left);
+    if ((tid & 63) == 0) todo[tid / 64] = m;
+    __syncthreads();
+    for (int wv = 0; wv < LSA_WAVES; ++wv) {
+      for (uint64_t left_m = todo[wv]; left_m; left_m &= left_m - 1) {  // uniform
+        const int64_t j = base + 64 * wv + (__ffsll((long long)left_m) - 1);
+        const int g = (int)(j % a.Hkv);
+        const int64_t x = j / a.Hkv, u = a.u0 + x / RT;
+        const int64_t b = u / a.n_rt, t = (u % a.n_rt) * RT + x % RT;
+        const int64_t li = list_of(a, b, t, g);
+        int n = a.lengths[li];
+        n = n < 0 ? 0 : (n > a.W ? a.W : n);
+        const int32_t* list = a.ids + li * a.W;
+        const T* kb = (const T*)a.k + b * a.kv_sb + g * a.kv_sh + lp * S::VEC;
+        const T* vb = (const T*)a.v + b * a.kv_sb + g * a.kv_sh + lp * S::VEC;
+        const int64_t qo = ((b * a.Tq + t) * a.Hq + (int64_t)g * GQ) * D;
+        AttnState<T, D, GQ> st;
+        attend_span<T, D, GQ>((const T*)a.q + qo, kb, vb, a.kv_st, a.Tk, 0, n,
+                              [&](int s) {
+                                const int32_t id = n > 0 ? list[s < n ? s : n - 1] : -1;
+                                return s < n ? id : -1;
+                              },
+                              a.scale_log2, st);
+        finish_span<T, D, GQ, kMaxSplits, true>(sh, st, true, (T*)a.out + qo, nullptr, a.empty_nan);
+        __syncthreads();  // sh is used again
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// ---------------------------------------------------------------- host
+
+struct Layout {
+  int gq, rb;
+  int64_t n_rt, n_tile, u_total, slab_u, blocks;
+  size_t bits, any, dup, rest, odd, total;
+};
+
+Layout layout_of(int64_t B, int64_t Tq, int64_t Tk, int32_t Hq, int32_t Hkv, int per_head) {
+  Layout l;
+  l.gq = Hq / Hkv;
+  l.rb = kWaves / l.gq;
+  l.n_rt = (Tq + l.rb * kBlockRows - 1) / (l.rb * kBlockRows);
+  l.n_tile = (Tk + kTile - 1) / kTile;
+  l.u_total = B * l.n_rt;
+  const int64_t per_u = (int64_t)l.rb * (per_head ? Hkv : 1);  // blocks a row tile
+  const int64_t fit = kSlabBytes / (per_u * l.n_tile * kBlockRows * 8);
+  l.slab_u = fit < 1 ? 1 : (fit < l.u_total ? fit : l.u_total);
+  l.blocks = l.slab_u * per_u;
+  auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };
+  l.bits = 0;
+  l.any = l.bits + up((size_t)l.blocks * l.n_tile * kBlockRows * 8);
+  l.dup = l.any + up((size_t)l.blocks * l.n_tile);
+  l.rest = l.dup + up((size_t)l.blocks * kBlockRows);
+  l.odd = l.rest + up((size_t)l.slab_u * Hkv);
+  l.total = l.odd + up((size_t)B * Hkv * l.n_tile);
+  return l;
+}
+
+template <typename T, int D, int GQ>
+void launch_slab(const RowsArgs& a, const Layout& l, hipStream_t s) {
+  const int64_t per_u = (int64_t)l.rb * (a.per_head ? a.Hkv : 1);
+  row_bits_kernel<<<dim3((unsigned)(a.n_u * per_u)), kBitThreads, 0, s>>>(a);
+  rows_mfma_kernel<T, D, GQ><<<dim3((unsigned)(a.n_u * a.Hkv)), kThreads, 0, s>>>(a);
+  const int64_t units = (int64_t)a.n_u * l.rb * kBlockRows * a.Hkv;
+  const int64_t blocks = (units + LSA_BLOCK - 1) / LSA_BLOCK;
+  rows_rest_kernel<T, D, GQ><<<dim3((unsigned)(blocks < 2048 ? blocks : 2048)), LSA_BLOCK, 0, s>>>(a);
+}
+
+template <typename T, int D>
+void launch_rows(RowsArgs a, const Layout& l, int64_t kv_batches, uint8_t* odd, hipStream_t s) {
+  tile_finite_kernel<T, D><<<dim3((unsigned)l.n_tile, (unsigned)a.Hkv, (unsigned)kv_batches), LSA_BLOCK, 0, s>>>(a, odd);
+  for (int64_t u = 0; u < l.u_total; u += l.slab_u) {
+    a.u0 = u;
+    a.n_u = (int)(l.u_total - u < l.slab_u ? l.u_total - u : l.slab_u);
+    switch (l.gq) {
+      case 1: launch_slab<T, D, 1>(a, l, s); break;
+      case 2: launch_slab<T, D, 2>(a, l, s); break;
+      case 4: launch_slab<T, D, 4>(a, l, s); break;
+      default: launch_slab<T, D, 8>(a, l, s); break;
+    }
+  }
+}
+
+bool rows_fit(int dtype, int64_t B, int64_t Tq, int64_t Tk, int32_t Hq, int32_t Hkv, int32_t D, int32_t W) {
+  if (!(dtype == LSA_BF16 || dtype == LSA_F16) || !(D == 64 || D == 128)) return false;
+  if (B < 1 || Tq < 1 || Tk < 1 || Hkv < 1 || Hq < Hkv || Hq % Hkv || W < 1) return false;
+  const int gq = Hq / Hkv;
+  if (!(gq == 1 || gq == 2 || gq == 4 || gq == 8)) return false;
+  return Tk <= (int64_t)kMaxTiles * kTile && B <= 65535 && Hkv <= 65535;
+}
+
+}  // namespace
+
+extern "C" size_t lsa_read_rows_scratch_bytes(int dtype, int64_t B, int64_t Tq, int64_t Tk, int32_t Hq, int32_t Hkv,
+                                              int32_t D, int32_t W, int ids_per_head) {
+  if (!rows_fit(dtype, B, Tq, Tk, Hq, Hkv, D, W)) return 0;
+  return layout_of(B, Tq, Tk, Hq, Hkv, ids_per_head ? 1 : 0).total;
+}
+
+extern "C" int lsa_read_rows(const void* q, const void* k, const void* v, int dtype, int64_t B, int64_t Tq, int64_t Tk,
+                             int32_t Hq, int32_t Hkv, int32_t D, int64_t kv_batch_stride, int64_t kv_token_stride,
+                             int64_t kv_head_stride, const int32_t* ids, const int32_t* lengths, int32_t W,
+                             int ids_per_head, float scale, int empty_nan, void* scratch, size_t scratch_bytes,
+                             void* out, void* stream) {
+  LSA_REQUIRE(q && k && v && ids && lengths && out, LSA_ERR_NULL, "lsa_read_rows: NULL pointer");
+  LSA_REQUIRE(rows_fit(dtype, B, Tq, Tk, Hq, Hkv, D, W), LSA_ERR_SHAPE, "lsa_read_rows: shape not served");
+  LSA_REQUIRE(scale > 0.0f && isfinite(scale), LSA_ERR_SHAPE, "lsa_read_rows: scale must be positive and finite");
+  const uintptr_t mis = ((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)out) & 15;
+  LSA_REQUIRE(mis == 0, LSA_ERR_ALIGN, "lsa_read_rows: q/k/v/out must be 16-byte aligned");
+  LSA_REQUIRE(kv_batch_stride >= 0 && kv_token_stride >= D && kv_head_stride >= D && kv_token_stride < (1 << 24),
+              LSA_ERR_SHAPE, "lsa_read_rows: K/V strides");
+  LSA_REQUIRE(((kv_batch_stride | kv_token_stride | kv_head_stride) * 2) % 16 == 0, LSA_ERR_ALIGN,
+              "lsa_read_rows: K/V strides must keep rows 16-byte aligned");
+  const Layout l = layout_of(B, Tq, Tk, Hq, Hkv, ids_per_head ? 1 : 0);
+  LSA_REQUIRE(scratch && ((uintptr_t)scratch & 255) == 0 && scratch_bytes >= l.total, LSA_ERR_WORKSPACE,
+              "lsa_read_rows: scratch %zu < %zu bytes", scratch_bytes, l.total);
+  LSA_REQUIRE(l.blocks <= 0x7FFFFFFF && l.slab_u * Hkv <= 0x7FFFFFFF, LSA_ERR_SHAPE, "lsa_read_rows: too many rows");
+  RowsArgs a;
+  char* ws = (char*)scratch;
+  a.q = q; a.k = k; a.v = v; a.out = out; a.ids = ids; a.lengths = lengths;
+  a.Tq = Tq; a.Tk = Tk; a.kv_sb = kv_batch_stride; a.kv_st = kv_token_stride; a.kv_sh = kv_head_stride;
+  a.Hq = Hq; a.Hkv = Hkv; a.W = W; a.per_head = ids_per_head ? 1 : 0;
+  a.u0 = 0; a.n_u = 0; a.n_rt = (int)l.n_rt; a.rb = l.rb; a.n_tile = (int)l.n_tile;
+  a.bits = (uint64_t*)(ws + l.bits); a.any = (uint8_t*)(ws + l.any); a.dup = (uint8_t*)(ws + l.dup);
+  a.rest = (uint8_t*)(ws + l.rest); a.odd = (const uint8_t*)(ws + l.odd);
+  a.scale_log2 = scale * kLog2e; a.empty_nan = empty_nan ? 1 : 0;
+  const int64_t kv_batches = kv_batch_stride ? B : 1;
+  uint8_t* odd = (uint8_t*)(ws + l.odd);
+  hipStream_t s = (hipStream_t)stream;
+  if (dtype == LSA_BF16) {
+    if (D == 64) launch_rows<bf16_t, 64>(a, l, kv_batches, odd, s);
+    else launch_rows<bf16_t, 128>(a, l, kv_batches, odd, s);
+  } else {
+    if (D == 64) launch_rows<_Float16, 64>(a, l, kv_batches, odd, s);
+    else launch_rows<_Float16, 128>(a, l, kv_batches, odd, s);
+  }
+  LSA_LAUNCHED("lsa_read_rows");
+  return LSA_OK;
+}

@@ -73,6 +73,9 @@ SIGNATURES = {
     "lsa_read_tile_tokens": (_i32, [_int, _i32, _i32]),
     "lsa_read": (_int, [_p, _p, _p, _int, _i64, _i64, _i64, _i32, _i32, _i32, _i64, _i64, _i64, _p, _p, _i32, _int,
                         _f32, _int, _i32, _p, _p, _sz, _p, _p]),
+    "lsa_read_rows_scratch_bytes": (_sz, [_int, _i64, _i64, _i64, _i32, _i32, _i32, _i32, _int]),
+    "lsa_read_rows": (_int, [_p, _p, _p, _int, _i64, _i64, _i64, _i32, _i32, _i32, _i64, _i64, _i64, _p, _p, _i32, _int,
+                             _f32, _int, _p, _sz, _p, _p]),
     "lsa_read_chunked": (_int, [_p, _p, _p, _int, _i64, _i64, _i64, _i32, _i32, _i32, _i64, _i64, _i64, _p, _p, _i32,
                                 _i32, _p, _f32, _i32, _p, _p]),
     "lsa_read_chunked_mfma_ok": (_int, [_int, _i32, _i32]),

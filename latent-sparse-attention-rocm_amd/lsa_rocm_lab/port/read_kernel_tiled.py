@@ -1,10 +1,12 @@
 """The sparse read (reference src/lsa_rocm_lab/port/read_kernel_tiled.py).
 
-One HIP gather-attention kernel serves every launch shape. A workgroup owns one
+One HIP gather-attention kernel serves any launch shape. A workgroup owns one
 (query row, kv-head) and a slice of its read list; the kv-head's whole GQA group
 shares each gathered K/V row, fetched once as 16-byte coalesced loads; scores and
 the online softmax are fp32; when there are few rows (decode) each list is split
-over several workgroups and the last one to finish merges their softmax partials.
+over several workgroups and the last one to finish merges their softmax partials. Many rows
+over one cache (a prefill's) go to a masked sweep on the matrix cores instead where that is
+faster (``_sweep_pays``).
 Contract as the reference: -1 ids and slots past a row's length are skipped,
 duplicates count per occurrence, a row with no keys gives zeros, the output has q's
 dtype. Lists are [B, Tq, W] shared by all heads or [B, Tq, Hkv, W] per kv-head
@@ -37,6 +39,36 @@ def _read_splits(units: int, width: int, tile: int) -> int:
         return max(1, min(int(env), MAX_SPLITS))
     tiles = max(1, math.ceil(width / tile))
     return max(1, min(tiles, max(1, 512 // max(units, 1)), MAX_SPLITS))
+
+
+# The gather's microseconds per (query row, kv-head, listed key) at head dim 128 and, by query
+# group, at 64 (measured on lists of 300 to 4300 keys, 1 to 8 kv-heads), and the sweep's per
+# 64-key tile of a workgroup.
+_GATHER_128 = 3.1e-5
+_GATHER_64 = {1: 1.07e-5, 2: 1.5e-5, 4: 2.3e-5, 8: 4.8e-5}
+_TILE_US = {64: 1.9, 128: 2.6}
+
+
+def _sweep_pays(dtype, B: int, Tq: int, Tk: int, Hq: int, Hkv: int, D: int, width: int, token_stride: int,
+                scale: float) -> bool:
+    """Whether a read goes to the masked sweep on the matrix cores (``lsa_read_rows``) rather
+    than the gather: the sweep's time follows the tiles its workgroups of 256 query columns
+    cross (on 256 CUs; the longest workgroup crosses the cache), the gather's the listed keys.
+    A row of a prefill lists about half of a short cache, ``width`` of a long one; lists are
+    not read here. 16-bit rows of head dim 64 or 128. At the reference's lists (Hq 32, Hkv 8, D 128) the gather
+    / the sweep take 65 / 60 us at 512 rows, 195 / 81 at 1024, 18.2 / 2.9 ms at 16384; at Hq 1,
+    Hkv 1, D 64 37 / 106 us at 2048, 346 / 311 at 8192."""
+    if dtype not in (torch.bfloat16, torch.float16) or D not in _TILE_US or not 0.0 < scale < math.inf:
+        return False
+    group = Hq // Hkv
+    if group not in _GATHER_64 or token_stride >= 1 << 24 or Tk < 1 or width < 1:
+        return False
+    tiles = -(-Tk // 64)
+    units = B * -(-Tq // (256 // group)) * Hkv
+    crossed = units * tiles * (0.6 if 2 * Tq > Tk else 1.0)  # a prefill's early rows see little
+    sweep = 50.0 + max(crossed / 256.0, float(tiles)) * _TILE_US[D] + B * Tq * width * 1e-6
+    gather = 20.0 + B * Tq * Hkv * min(width, 0.45 * Tk) * (_GATHER_128 if D == 128 else _GATHER_64[group])
+    return sweep < gather
 
 
 def _kv_layout(k: torch.Tensor, v: torch.Tensor):
@@ -73,6 +105,16 @@ def _sparse_read(q, k, v, read_ids, lengths, scale, empty_nan: bool, splits: int
     out = torch.empty_like(q)
     if rows == 0:
         return out
+    scale = float(D ** -0.5 if scale is None else scale)
+    if splits is None and _sweep_pays(q.dtype, B, Tq, Tk, Hq, Hkv, D, width, st, scale):
+        nbytes = _abi.size("lsa_read_rows_scratch_bytes", _abi.dtype_code(q.dtype), B, Tq, Tk, Hq, Hkv, D, width,
+                           1 if per_head else 0)
+        if nbytes > 0:
+            ws = _abi.Workspace.get(q.device, "read_rows", nbytes)
+            _abi.call("lsa_read_rows", q.data_ptr(), k.data_ptr(), v.data_ptr(), _abi.dtype_code(q.dtype), B, Tq, Tk,
+                      Hq, Hkv, D, sb, st, sh, ids.data_ptr(), lens.data_ptr(), width, 1 if per_head else 0, scale,
+                      1 if empty_nan else 0, ws.data_ptr(), nbytes, out.data_ptr(), _abi.stream(q.device))
+            return out
     if splits is None:
         tile = _abi.size("lsa_read_tile_tokens", _abi.dtype_code(q.dtype), D, Hq // Hkv)
         splits = _read_splits(rows * Hkv, width, max(tile, 1))
@@ -80,7 +122,7 @@ def _sparse_read(q, k, v, read_ids, lengths, scale, empty_nan: bool, splits: int
     ws = _abi.Workspace.get(q.device, "read", nbytes)
     counters = _abi.Counters.get(q.device, rows * Hkv) if nbytes else None
     _abi.call("lsa_read", q.data_ptr(), k.data_ptr(), v.data_ptr(), _abi.dtype_code(q.dtype), B, Tq, Tk, Hq, Hkv, D,
-              sb, st, sh, ids.data_ptr(), lens.data_ptr(), width, 1 if per_head else 0, float(D ** -0.5 if scale is None else scale),
+              sb, st, sh, ids.data_ptr(), lens.data_ptr(), width, 1 if per_head else 0, scale,
               1 if empty_nan else 0, splits, _abi.ptr(counters), _abi.ptr(ws), nbytes, out.data_ptr(),
               _abi.stream(q.device))
     return out

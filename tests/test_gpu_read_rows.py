@@ -1,0 +1,147 @@
+"""The per-row read as a masked sweep on the matrix cores (lsa_read_rows) vs the fp64 oracle.
+
+Cases at the kernel's edges: row counts and caches around its tiles (32-row blocks, 64-key
+tiles, 256 columns), both 16-bit types, head dims 64 and 128, query groups 1, 2, 4 and 8,
+shared and per-kv-head lists, several batch rows and one pool for all of them, skipped ids,
+ids listed twice (those rows go to the gather), rows with nothing to read under both
+contracts, K/V values that are not finite (listed and not), lists too sparse for the sweep,
+caches long enough for several bitmap segments and several slabs of rows.
+
+Bound: the output's own rounding (2^-9 of it in bf16, 2^-12 in fp16, doubled), plus 2^-13 of
+the largest |v| for the split weights (2^-16) and the fp32 scores of up to 128 products.
+"""
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from lsa_rocm_lab import _abi
+from lsa_rocm_lab.port.read_kernel_tiled import _sparse_read
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+RTOL = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}
+
+
+def make(dtype, B, Tq, Tk, Hq, Hkv, D, W, per_head=False, seed=0, short=1.0, pool=False):
+    """q, k, v and distinct ids in a random order, -1 and out-of-range ids among them, every
+    17th list empty."""
+    g = torch.Generator().manual_seed(seed)
+    q = torch.randn(B, Tq, Hq, D, generator=g).to(dtype)
+    k = torch.randn(1 if pool else B, Tk, Hkv, D, generator=g).to(dtype)
+    v = torch.randn(1 if pool else B, Tk, Hkv, D, generator=g).to(dtype)
+    shape = (B, Tq, Hkv) if per_head else (B, Tq)
+    n = int(np.prod(shape))
+    rng = np.random.default_rng(seed)
+    ids = np.full((n, W), -1, np.int32)
+    for i in range(n):
+        m = min(W, Tk)
+        ids[i, :m] = rng.permutation(Tk)[:m]
+    ids[:, 5::13] = -1
+    ids[::7, 0] = Tk + 3
+    lengths = rng.integers(0, max(1, int(W * short)) + 1, n).astype(np.int32)
+    lengths[::17] = 0
+    return q, k, v, torch.from_numpy(ids.reshape(*shape, W)), torch.from_numpy(lengths.reshape(shape))
+
+
+def sweep(q, k, v, ids, lengths, empty_nan=False, scale=None):
+    B, Tq, Hq, D = q.shape
+    Tk, Hkv = k.shape[1:3]
+    per_head = ids.dim() == 4
+    args = [t.to(DEV).contiguous() for t in (q, k, v, ids, lengths)]
+    dt, W = _abi.dtype_code(q.dtype), ids.shape[-1]
+    nbytes = _abi.size("lsa_read_rows_scratch_bytes", dt, B, Tq, Tk, Hq, Hkv, D, W, int(per_head))
+    assert nbytes > 0
+    ws = torch.full((nbytes,), 0xA5, dtype=torch.uint8, device=DEV)  # needs no initialisation
+    out = torch.full_like(args[0], float("nan"))
+    sb = args[1].stride(0) if k.shape[0] == B else 0
+    print(f"rows sweep q={tuple(q.shape)} {q.dtype} Tk={Tk} Hkv={Hkv} W={W} per_head={per_head}", flush=True)
+    _abi.call("lsa_read_rows", args[0].data_ptr(), args[1].data_ptr(), args[2].data_ptr(), dt, B, Tq, Tk, Hq, Hkv, D,
+              sb, args[1].stride(1), args[1].stride(2), args[3].data_ptr(), args[4].data_ptr(), W, int(per_head),
+              float(D ** -0.5 if scale is None else scale), int(empty_nan), ws.data_ptr(), nbytes, out.data_ptr(),
+              _abi.stream(out.device))
+    torch.cuda.synchronize()
+    return out
+
+
+def check(q, k, v, ids, lengths, empty_nan=False, rows=None):
+    got = sweep(q, k, v, ids, lengths, empty_nan).float().cpu().numpy()
+    kk, vv = (t.expand(q.shape[0], *t.shape[1:]).float().numpy() for t in (k, v))
+    idn = ids.numpy().copy()
+    idn[idn >= k.shape[1]] = -1  # the oracle indexes rows; out-of-range ids are skipped like -1
+    pick = slice(None) if rows is None else rows
+    want = oracle.sparse_read(q[:, pick].float().numpy(), kk, vv, idn[:, pick], lengths.numpy()[:, pick],
+                              empty="nan" if empty_nan else "zero")
+    got = got[:, pick]
+    assert np.array_equal(np.isfinite(got), np.isfinite(want))
+    ok = np.isfinite(want)
+    bound = RTOL[q.dtype] * np.abs(want[ok]) + 2.0 ** -13 * float(np.nanmax(np.abs(vv[np.isfinite(vv)])))
+    err = np.abs(got[ok] - want[ok])
+    assert (err <= bound).all(), (err.max(), (err - bound).max())
+
+
+@pytest.mark.parametrize("dtype,B,Tq,Tk,Hq,Hkv,D,W,per_head", [
+    (torch.bfloat16, 1, 1, 1, 8, 2, 128, 4, False),        # one row, one key
+    (torch.bfloat16, 1, 31, 63, 4, 1, 64, 63, False),      # one key short of a tile, a row short of a block
+    (torch.float16, 1, 33, 65, 8, 1, 128, 65, False),      # one past
+    (torch.bfloat16, 2, 64, 256, 8, 8, 128, 200, False),   # query group 1: 256 rows a workgroup
+    (torch.float16, 2, 129, 321, 4, 2, 64, 321, True),     # group 2, a list a kv-head
+    (torch.bfloat16, 1, 300, 517, 32, 8, 128, 517, False),  # group 4
+    (torch.bfloat16, 1, 70, 640, 8, 1, 64, 600, False),    # group 8: 32 rows a workgroup
+    (torch.float16, 1, 97, 130, 2, 2, 64, 130, True),
+])
+def test_edges_vs_oracle(dtype, B, Tq, Tk, Hq, Hkv, D, W, per_head):
+    check(*make(dtype, B, Tq, Tk, Hq, Hkv, D, W, per_head, seed=Tq))
+
+
+@pytest.mark.parametrize("empty_nan", [False, True])
+def test_duplicates_and_empty_rows(empty_nan):
+    q, k, v, ids, lengths = make(torch.bfloat16, 1, 96, 300, 8, 2, 128, 300, seed=3)
+    ids[:, ::5, 1:3] = ids[:, ::5, 3:4]  # counted per occurrence
+    check(q, k, v, ids, lengths, empty_nan)
+
+
+def test_values_that_are_not_finite():
+    """A NaN K row and an infinite V row: rows that list the NaN row as the gather reads them,
+    every other row untouched by either (the tile's workgroups go to the gather)."""
+    q, k, v, ids, lengths = make(torch.bfloat16, 1, 96, 400, 8, 2, 64, 200, seed=4)
+    k[0, 130, 0] = float("nan")
+    v[0, 390, 1] = float("inf")
+    lists = ids.numpy()[0]
+    hit = np.array([(lists[t, : int(lengths[0, t])] == 130).any() for t in range(96)])
+    got = sweep(q, k, v, ids, lengths)
+    dev = [t.to(DEV) for t in (q, k, v, ids, lengths)]
+    gathered = _sparse_read(*dev, None, False, splits=1)
+    assert hit.any() and torch.equal(got[0, torch.from_numpy(hit)], gathered[0, torch.from_numpy(hit)])
+    clean = np.nonzero(~hit & ~np.array([(lists[t, : int(lengths[0, t])] == 390).any() for t in range(96)]))[0]
+    want = oracle.sparse_read(q[:, clean].float().numpy(), np.nan_to_num(k.float().numpy()),
+                              np.nan_to_num(v.float().numpy(), posinf=0.0), np.where(lists >= 400, -1, lists)[None][:, clean],
+                              lengths.numpy()[:, clean])
+    assert np.abs(got[:, clean].float().cpu().numpy() - want).max() <= 2.0 ** -8 * np.abs(want).max() + 2.0 ** -11
+
+
+def test_sparse_lists_and_one_pool():
+    """A few keys a row over a long cache (left to the gather), K/V one pool of both rows."""
+    check(*make(torch.bfloat16, 2, 80, 5000, 8, 1, 128, 40, seed=5, short=0.2, pool=True))
+
+
+def test_large_scores():
+    """Scores of a wide spread: the running maximum moves in steps, weights of 2^-100 beside 1."""
+    q, k, v, ids, lengths = make(torch.float16, 1, 64, 500, 4, 1, 128, 500, seed=6)
+    check(q * 6, k * 4, v, ids, lengths)
+
+
+def test_segments_and_slabs():
+    """A 262144-row cache (eight bitmap segments, a slab of 64 row tiles) under 2080 rows: both
+    slabs' rows against the oracle, keys of every segment."""
+    B, Tq, Tk, Hq, Hkv, D, W = 1, 2080, 262144, 8, 1, 64, 200
+    g = torch.Generator().manual_seed(7)
+    q = torch.randn(B, Tq, Hq, D, generator=g).half()
+    k, v = (torch.randn(B, Tk, Hkv, D, generator=g).half() for _ in range(2))
+    # dense at the end (dense enough for the sweep), a key in every segment
+    pick = torch.stack([torch.randperm(512, generator=g)[:192] for _ in range(Tq)])
+    ids = torch.cat([pick + (Tk - 512), torch.arange(8).expand(Tq, 8) * 32768 + 5], 1).int()[None]
+    lengths = torch.full((B, Tq), W, dtype=torch.int32)
+    rows = [0, 31, 32, 1000, 2047, 2048, 2079]
+    check(q, k, v, ids, lengths, rows=rows)
