@@ -429,6 +429,25 @@ template <typename QT, int V> struct RowVec;
 template <typename QT> struct RowVec<QT, 1> {
   static __device__ __forceinline__ void load(const QT* p, float* f) { f[0] = elem<QT>::load(p, 0); }
 };
+template <> struct RowVec<float, 2> {
+  static __device__ __forceinline__ void load(const float* p, float* f) {
+    const float2 x = *(const float2*)p;
+    f[0] = x.x; f[1] = x.y;
+  }
+};
+template <> struct RowVec<bf16_t, 2> {
+  static __device__ __forceinline__ void load(const bf16_t* p, float* f) {
+    const uint32_t x = *(const uint32_t*)p;
+    f[0] = __uint_as_float(x << 16); f[1] = __uint_as_float(x & 0xFFFF0000u);
+  }
+};
+template <> struct RowVec<_Float16, 2> {
+  static __device__ __forceinline__ void load(const _Float16* p, float* f) {
+    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+    const h2 x = *(const h2*)p;
+    f[0] = (float)x[0]; f[1] = (float)x[1];
+  }
+};
 template <> struct RowVec<float, 4> {
   static __device__ __forceinline__ void load(const float* p, float* f) {
     const float4 x = *(const float4*)p;
@@ -495,39 +514,73 @@ __global__ void index_queries_kernel(const QT* q, int64_t B, int64_t T, int Hq, 
   for (int e = 0; e < V; ++e) out[idx * V + e] = acc[e] / cnt;
 }
 
-template <typename KT>
+// One wave a bucket: 64 member ids in one load, the valid ones taken in member order eight at a
+// time (their key rows all in flight, then added in order: the fp32 sum's definition), V dims a
+// lane. Latency-bound: 4096 buckets of ~64 keys in rows of 256 slots (32k positions, 8 kv-heads, D 128)
+// 161 -> 24 us, against a workgroup a bucket that walked every slot, padding included, one key
+// row in flight.
+template <typename KT, int V>
 __global__ __launch_bounds__(LSA_BLOCK) void centroids_kernel(const KT* keys, int64_t tokens, int64_t token_stride,
                                                               int64_t batch_stride, int kv_heads, int D,
-                                                              const int32_t* members, int rows, int cap,
-                                                              int mode, float* out_f32, uint16_t* out_bf16) {
-  __shared__ float sums[512];
-  __shared__ float norm;
-  const int64_t bucket = blockIdx.x;
+                                                              const int32_t* members, int64_t buckets, int rows,
+                                                              int cap, int mode, float* out_f32, uint16_t* out_bf16) {
+  constexpr int NB = 8;
+  __shared__ float sums[LSA_WAVES][512];
+  const int lane = threadIdx.x & (LSA_WAVE - 1), w = threadIdx.x / LSA_WAVE;
+  const int64_t bucket = (int64_t)blockIdx.x * LSA_WAVES + w;
+  if (bucket >= buckets) return;  // the whole wave; no barrier follows
   const int64_t table = bucket / rows;
   const KT* kb = keys + (table / kv_heads) * batch_stride + (table % kv_heads) * (int64_t)D;
   const int32_t* m = members + bucket * cap;
   int count = 0;
-  for (int j = 0; j < cap; ++j) count += (m[j] >= 0 && m[j] < tokens) ? 1 : 0;
-  for (int d = threadIdx.x; d < D; d += LSA_BLOCK) {
-    float acc = 0.0f;
-    for (int j = 0; j < cap; ++j) {
-      const int32_t id = m[j];
-      if (id >= 0 && id < tokens) acc += elem<KT>::load(kb, (int64_t)id * token_stride + d);
+  for (int d0 = 0; d0 < D; d0 += V * LSA_WAVE) {
+    const int d = d0 + V * lane;
+    const KT* kd = kb + (d < D ? d : 0);
+    float acc[V];
+#pragma unroll
+    for (int e = 0; e < V; ++e) acc[e] = 0.0f;
+    count = 0;
+    for (int j0 = 0; j0 < cap; j0 += LSA_WAVE) {
+      const int32_t id = j0 + lane < cap ? m[j0 + lane] : -1;
+      uint64_t left = __ballot(id >= 0 && id < tokens);
+      count += __popcll(left);
+      while (left) {  // uniform
+        const int n = __popcll(left);
+        float x[NB][V];
+#pragma unroll
+        for (int u = 0; u < NB; ++u) {  // past the last member its row again, not added
+          const int32_t row = __builtin_amdgcn_readlane(id, __ffsll((long long)left) - 1);
+          RowVec<KT, V>::load(kd + (int64_t)row * token_stride, x[u]);
+          const uint64_t rest = left & (left - 1);
+          left = rest ? rest : left;
+        }
+#pragma unroll
+        for (int u = 0; u < NB; ++u) {
+          if (u < n) {
+#pragma unroll
+            for (int e = 0; e < V; ++e) acc[e] += x[u][e];
+          }
+        }
+        if (n <= NB) left = 0;
+      }
     }
-    sums[d] = acc;
+    if (d < D) {
+#pragma unroll
+      for (int e = 0; e < V; ++e) sums[w][d + e] = acc[e];
+    }
   }
-  __syncthreads();
-  if (mode == LSA_CENTROID_NORMALIZED && threadIdx.x == 0) {
+  __builtin_amdgcn_wave_barrier();  // the wave's LDS writes before its reads
+  float norm = 1.0f;
+  if (mode == LSA_CENTROID_NORMALIZED) {  // the fp64 square sum in the order of the dims
     double sq = 0.0;
-    for (int d = 0; d < D; ++d) sq += (double)sums[d] * (double)sums[d];
+    for (int d = 0; d < D; ++d) sq += (double)sums[w][d] * (double)sums[w][d];
     norm = fmaxf((float)sqrt(sq), 1e-12f);
   }
-  __syncthreads();
-  for (int d = threadIdx.x; d < D; d += LSA_BLOCK) {
+  for (int d = lane; d < D; d += LSA_WAVE) {
     float c;
-    if (mode == LSA_CENTROID_NORMALIZED) c = sums[d] / norm;
-    else if (mode == LSA_CENTROID_SUM) c = sums[d];
-    else c = count > 0 ? sums[d] / (float)count : 0.0f;
+    if (mode == LSA_CENTROID_NORMALIZED) c = sums[w][d] / norm;
+    else if (mode == LSA_CENTROID_SUM) c = sums[w][d];
+    else c = count > 0 ? sums[w][d] / (float)count : 0.0f;
     out_f32[bucket * D + d] = c;
     if (out_bf16) out_bf16[bucket * D + d] = f32_to_bf16(c);
   }
@@ -858,11 +911,18 @@ extern "C" int lsa_bucket_centroids(const void* keys, int k_dtype, int64_t token
   if (n == 0) return LSA_OK;
   LSA_REQUIRE(n <= 0x7FFFFFFF, LSA_ERR_SHAPE, "lsa_bucket_centroids: too many buckets");
   hipStream_t s = (hipStream_t)stream;
+  // pairs of dims a lane where a pair of every row is one aligned load and the rows fill the lanes
+  const int esize = k_dtype == LSA_F32 ? 4 : 2;
+  const bool pairs = D % 2 == 0 && D > LSA_WAVE && token_stride % 2 == 0 && batch_stride % 2 == 0 &&
+                     ((uintptr_t)keys % (2 * esize)) == 0;
+  const dim3 grid((unsigned)((n + LSA_WAVES - 1) / LSA_WAVES));
   LSA_DISPATCH_QT(k_dtype, {
-    centroids_kernel<QT><<<dim3((unsigned)n), LSA_BLOCK, 0, s>>>((const QT*)keys, tokens, token_stride, batch_stride,
-                                                                kv_heads,
-                                                                D, members, rows, cap, centroid_mode, out_f32,
-                                                                out_bf16);
+    if (pairs)
+      centroids_kernel<QT, 2><<<grid, LSA_BLOCK, 0, s>>>((const QT*)keys, tokens, token_stride, batch_stride, kv_heads,
+                                                        D, members, n, rows, cap, centroid_mode, out_f32, out_bf16);
+    else
+      centroids_kernel<QT, 1><<<grid, LSA_BLOCK, 0, s>>>((const QT*)keys, tokens, token_stride, batch_stride, kv_heads,
+                                                        D, members, n, rows, cap, centroid_mode, out_f32, out_bf16);
   })
   LSA_LAUNCHED("lsa_bucket_centroids");
   return LSA_OK;
