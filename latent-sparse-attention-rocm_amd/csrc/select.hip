@@ -471,10 +471,14 @@ template <> struct RowVec<_Float16, 4> {
 
 // One thread per V dims of an output row (b, chunk, kv-head): the fp32 sum over the
 // chunk's tokens and, within a token, the group's heads in order (the canonical order),
-// then one division. The (token, head) rows are walked in batches of 16 whose loads are
-// all in flight before the batch's adds.
-template <typename QT, int V>
-__global__ void index_queries_kernel(const QT* q, int64_t B, int64_t T, int Hq, int Hkv, int D, int chunk,
+// then one division. The (token, head) rows are walked in batches of NB whose loads are
+// all in flight before the batch's adds. GC: the group's size where it divides NB (a batch is
+// whole tokens), 0: any (a row's place is then ~25 scalar operations, which over 256 rows are
+// 10 us). Memory-bound with many rows (32k tokens of 32 heads, D 128: 58.3 -> 48.3 us, 5.6 TB/s);
+// with few, the batches are a chain of round trips: 78 chunks of 64 x 4 rows, 4 kv-heads, D 64
+// 30.1 -> 8.3 us (V 4, NB 16 -> V 1, NB 64).
+template <typename QT, int V, int NB, int GC>
+__global__ __launch_bounds__(256) void index_queries_kernel(const QT* q, int64_t B, int64_t T, int Hq, int Hkv, int D, int chunk,
                                      float* out) {
   const int64_t C = T / chunk;
   const int DV = D / V;
@@ -489,18 +493,32 @@ __global__ void index_queries_kernel(const QT* q, int64_t B, int64_t T, int Hq, 
   const QT* base = q + ((b * T + c * chunk) * Hq + (int64_t)g * G) * D + dv * V;
   const int64_t tstride = (int64_t)Hq * D;
   const int rows = chunk * G;  // (token, head) rows, token-major
-  constexpr int NB = 16;
   float acc[V];
 #pragma unroll
   for (int e = 0; e < V; ++e) acc[e] = 0.0f;
+  int h = 0;
+  int64_t off = 0;  // of the next row (GC 0) or token
   for (int k0 = 0; k0 < rows; k0 += NB) {
     float x[NB][V];
+    // past the last row its loads repeat: every load in bounds (no branch: the loads stay together)
+    if constexpr (GC > 0) {
 #pragma unroll
-    for (int j = 0; j < NB; ++j) {
-      const int k = k0 + j < rows ? k0 + j : rows - 1;  // clamped: every load in bounds
-      const int t = k / G, h = k - t * G;
-      RowVec<QT, V>::load(base + t * tstride + (int64_t)h * D, x[j]);
+      for (int j = 0; j < NB; j += GC) {
+        const QT* p = base + off;
+#pragma unroll
+        for (int e = 0; e < GC; ++e) RowVec<QT, V>::load(p + e * D, x[j + e]);
+        off += -(int64_t)(k0 + j + GC < rows) & tstride;
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        RowVec<QT, V>::load(base + off, x[j]);
+        const int more = -(int)(k0 + j + 1 < rows), next = -(int)(h + 1 == G);
+        off += ((int64_t)more & D) + ((int64_t)(more & next) & (tstride - (int64_t)G * D));
+        h = (h - more) & ~(more & next);
+      }
     }
+    __builtin_amdgcn_sched_barrier(0);  // the adds stay behind the whole batch
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
       if (k0 + j < rows) {
@@ -880,15 +898,38 @@ extern "C" int lsa_index_queries(const void* q, int q_dtype, int64_t B, int64_t 
   if (n == 0) return LSA_OK;
   hipStream_t s = (hipStream_t)stream;
   const int esize = q_dtype == LSA_F32 ? 4 : 2;
-  const bool vec = D % 4 == 0 && ((uintptr_t)q % (4 * esize)) == 0;  // 4 dims a thread
-  const dim3 grid((unsigned)((n / (vec ? 4 : 1) + 255) / 256));
-  if (vec) {
-    LSA_DISPATCH_QT(q_dtype,
-                    { index_queries_kernel<QT, 4><<<grid, 256, 0, s>>>((const QT*)q, B, T, Hq, Hkv, D, chunk, out); })
-  } else {
-    LSA_DISPATCH_QT(q_dtype,
-                    { index_queries_kernel<QT, 1><<<grid, 256, 0, s>>>((const QT*)q, B, T, Hq, Hkv, D, chunk, out); })
+  // dims a thread: 4 where aligned and the waves still cover the chip (4 a CU), else fewer, each
+  // with as many elements in flight; batches no longer than the rows
+  auto fits = [&](int v) { return D % v == 0 && ((uintptr_t)q % (v * esize)) == 0; };
+  const int64_t rows = (int64_t)chunk * (Hq / Hkv), few = 1024 * LSA_WAVE;
+  const int v = fits(4) && (n / 4 >= few || rows <= 16) ? 4 : (fits(2) && n / 2 >= few && rows > 16 ? 2 : 1);
+  const int threads = n / v >= few ? 256 : LSA_WAVE;
+  const dim3 grid((unsigned)((n / v + threads - 1) / threads));
+#define LSA_INDEX_QUERIES(V, NB, GC)                                                                         \
+  LSA_DISPATCH_QT(q_dtype, {                                                                                 \
+    index_queries_kernel<QT, V, NB, GC><<<grid, threads, 0, s>>>((const QT*)q, B, T, Hq, Hkv, D, chunk, out); \
+  })
+#define LSA_INDEX_QUERIES_G(V, NB)                 \
+  switch (Hq / Hkv) {                              \
+    case 1: LSA_INDEX_QUERIES(V, NB, 1) break;     \
+    case 2: LSA_INDEX_QUERIES(V, NB, 2) break;     \
+    case 4: LSA_INDEX_QUERIES(V, NB, 4) break;     \
+    case 8: LSA_INDEX_QUERIES(V, NB, 8) break;     \
+    default: LSA_INDEX_QUERIES(V, NB, 0) break;    \
   }
+  if (v == 4 && rows <= 4) {
+    LSA_INDEX_QUERIES(4, 4, 0)
+  } else if (v == 4) {
+    LSA_INDEX_QUERIES_G(4, 16)
+  } else if (v == 2) {
+    LSA_INDEX_QUERIES_G(2, 32)
+  } else if (rows <= 16) {
+    LSA_INDEX_QUERIES(1, 16, 0)
+  } else {
+    LSA_INDEX_QUERIES_G(1, 64)
+  }
+#undef LSA_INDEX_QUERIES_G
+#undef LSA_INDEX_QUERIES
   LSA_LAUNCHED("lsa_index_queries");
   return LSA_OK;
 }
