@@ -126,6 +126,22 @@ int lsa_select_flat(const void* queries, int q_dtype, int64_t R, int32_t G, int3
                     int32_t top_k, int32_t splits, int32_t* counters, void* scratch, size_t scratch_bytes,
                     int32_t* lists, int32_t* lengths, void* stream);
 
+/* The flat select of many query rows against one table a group (a prefill's): the scores of 16
+ * rows x 16 buckets as one fp64 matrix product, then a row's top-k and expansion from them.
+ * Lists and lengths identical to lsa_select_flat's: sums of bf16 products that fp64 may not
+ * hold exactly are made in the canonical order. Arguments as lsa_select_flat's with row_tables 0 and
+ * one split; head dim 64 or 128, score_mode LSA_SCORE_BF16, queries and centroids 16-byte
+ * aligned. lsa_select_rows_scratch_bytes(): 0 where it does not apply; scratch 16-byte aligned,
+ * no initialisation. */
+size_t lsa_select_rows_scratch_bytes(int64_t R, int32_t G, int32_t D, int32_t rows, int32_t top_p, int64_t row_tables,
+                                     int score_mode);
+int lsa_select_rows(const void* queries, int q_dtype, int64_t R, int32_t G, int32_t D, const void* centroids,
+                    const int32_t* members, const int32_t* ends, int32_t table_flags, int32_t rows, int32_t cap,
+                    int64_t group_tables, int score_mode, const int32_t* positions, const lsa_slot_map* slots,
+                    int32_t cluster_block_size, int32_t block_buckets, int32_t top_p, int32_t window, int32_t sink,
+                    int32_t top_k, void* scratch, size_t scratch_bytes, int32_t* lists, int32_t* lengths,
+                    void* stream);
+
 /* Two-level tree select (reference pipeline.py:319-337 tree_select, _tree.py:318-373
  * _beam_pick_rows with one node level, _tree.py:100-142 _growth_replay): per (row, group)
  * with V visible buckets, node growth covers the first C = min(floor(V / node_block) *

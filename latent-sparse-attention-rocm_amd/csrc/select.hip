@@ -269,6 +269,192 @@ __global__ __launch_bounds__(LSA_BLOCK) __attribute__((amdgpu_waves_per_eu(4, 4)
   expand_row(a, pk, t, ends, position, i, scan);
 }
 
+// ------------------------------------------------------------------ flat select of many rows
+//
+// A prefill selects for thousands of query rows against one table. A workgroup a row scores the
+// table for itself: every centroid element is converted to fp64 and every score folded over 16
+// lanes once a row, ~32 of the 40 us a CU spent on a row of 4096 buckets at D 128. Here the
+// scores of 16 rows x 16 buckets are one fp64 matrix product (v_mfma_f64_16x16x4, 32 of them at D
+// 128), written to scratch as fp32, and select_scored_kernel takes a row's scores from there; only
+// buckets a row sees are scored and ranked. 32k rows of 4096 buckets, 1024 picks, D 128: 5.18 ->
+// 1.34 ms (scores 0.42, picks and lists 0.86); 512 rows x 8 groups of 512 buckets, 32 picks: 102 ->
+// 72 us, where a screen on the bf16 matrix cores scored the table before.
+//
+// The canonical score is an fp64 sum in a fixed order, rounded to fp32 once. The operands are
+// bf16: a product has at most 16 bits, and with the elements' exponents (zeros aside) within
+// [qmin, qmax] and [cmin, cmax] every partial sum in any order is a multiple of
+// 2^(qmin + cmin - 14) below D * 2^(qmax + cmax + 2). That is exact in 53 bits if (qmax - qmin) +
+// (cmax - cmin) <= 37 - log2 D, so the order does not matter and the score is the canonical one,
+// bit for bit. The other pairs (3.5e-4 of them for normal draws at D 128; every pair of a row or a
+// bucket that is not finite) are scored in the canonical order by the wave that meets them.
+
+constexpr int kTileWaves = LSA_BLOCK / LSA_WAVE;
+
+// The exponent range of the bf16 numbers seen by the four lanes that share a row (lane % 16), each
+// holding some of its dims: `mx` their largest magnitude, `mn` the smallest of magnitude - 1 in
+// 16 bits (0 wraps to the largest). A value that is not finite gives a range no bound allows.
+__device__ __forceinline__ int exponent_range(uint32_t mx, uint32_t mn) {
+#pragma unroll
+  for (int x = 16; x <= 32; x *= 2) {
+    mx = max(mx, (uint32_t)__shfl_xor((int)mx, x));
+    mn = min(mn, (uint32_t)__shfl_xor((int)mn, x));
+  }
+  if ((mx >> 7) == 255) return 1 << 16;
+  if (mx == 0) return 0;
+  return (int)max(mx >> 7, 1u) - (int)max((mn + 1) >> 7, 1u);  // subnormals: the exponent of field 1
+}
+
+// grid (16-row tiles of [r0, R) x G, splits of the buckets). A wave holds 16 query rows in
+// registers as doubles (lane: row lane % 16, a quarter of its dims) and walks the 16-bucket tiles
+// any of them sees, the next tile's rows in flight. Bound by the fp64 matrix rate.
+template <typename QT, int D>
+__global__ __launch_bounds__(LSA_BLOCK) void score_tiles_kernel(const QT* q, FlatArgs a, int64_t r0, int64_t r1,
+                                                                float* scores) {
+  constexpr int KD = D / 4, SPAN = D / 16;
+  constexpr int LIMIT = 53 - 16 - (D == 128 ? 7 : 6);
+  typedef double f64x4_t __attribute__((ext_vector_type(4)));
+  typedef unsigned short u16x2_t __attribute__((ext_vector_type(2)));
+  const int lane = threadIdx.x & 63, w = threadIdx.x / 64, ln = lane & 15, kg = lane >> 4;
+  const int64_t g = blockIdx.x % a.G;
+  const int64_t rt = r0 + (int64_t)(blockIdx.x / a.G) * 16;  // the tile's first row
+  const bf16_t* cent = (const bf16_t*)a.centroids + g * a.group_tables * a.rows * (int64_t)D;
+  const int64_t my = min(rt + ln, r1 - 1);
+
+  double qd[KD];
+  int qrange[4];  // of rows rt + kg + 4 e, the rows of this lane's results
+  {
+    SpanRaw<QT, KD> raw;
+    raw.load(q + (my * a.G + g) * D + kg * KD);
+    uint32_t mx = 0, mn = 0xFFFF;
+#pragma unroll
+    for (int e = 0; e < KD; ++e) {
+      const float x = bf16_round(raw.at(e));
+      const uint32_t m = (__float_as_uint(x) >> 16) & 0x7FFFu;
+      mx = max(mx, m);
+      mn = min(mn, (m - 1) & 0xFFFFu);
+      qd[e] = (double)x;
+    }
+    const int range = exponent_range(mx, mn);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) qrange[e] = __shfl(range, kg + 4 * e);
+  }
+  int seen = a.rows;  // buckets any row of the tile sees (without span ends: a prefix)
+  if (!a.vends) {
+    seen = max(visible_closed(a.positions[my], a.rows, a.cluster_block, a.block_buckets), 0);
+#pragma unroll
+    for (int x = 1; x <= 8; x *= 2) seen = max(seen, __shfl_xor(seen, x));
+  }
+  const int tiles = __builtin_amdgcn_readfirstlane((seen + 15) / 16);
+  const int step = kTileWaves * (int)gridDim.y;
+  const auto row_of = [&](int tile) { return cent + (int64_t)min(tile * 16 + ln, a.rows - 1) * D + kg * KD; };
+
+  int tile = (int)blockIdx.y * kTileWaves + w;
+  SpanRaw<bf16_t, KD> raw, next;
+  if (tile < tiles) next.load(row_of(tile));
+  for (; tile < tiles; tile += step) {  // uniform in a wave; no barrier inside
+    raw = next;
+    next.load(row_of(min(tile + step, tiles - 1)));
+    u16x2_t mx2 = {0, 0}, mn2 = {0xFFFF, 0xFFFF};
+#pragma unroll
+    for (int e = 0; e < KD / 2; ++e) {
+      const u16x2_t m = __builtin_bit_cast(u16x2_t, raw.w[e] & 0x7FFF7FFFu);
+      mx2 = __builtin_elementwise_max(mx2, m);
+      mn2 = __builtin_elementwise_min(mn2, (u16x2_t)(m - (u16x2_t){1, 1}));
+    }
+    const int crange = exponent_range(max(mx2.x, mx2.y), min(mn2.x, mn2.y));
+    f64x4_t s0 = {0.0, 0.0, 0.0, 0.0}, s1 = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int e = 0; e < KD; e += 2) {
+      s0 = __builtin_amdgcn_mfma_f64_16x16x4f64(qd[e], (double)raw.at(e), s0, 0, 0, 0);
+      s1 = __builtin_amdgcn_mfma_f64_16x16x4f64(qd[e + 1], (double)raw.at(e + 1), s1, 0, 0, 0);
+    }
+    // lane: bucket 16 tile + ln, rows rt + kg + 4 e
+    const int col = tile * 16 + ln;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int64_t r = rt + kg + 4 * e;
+      const bool live = r < r1 && col < a.rows;
+      float s = (float)(s0[e] + s1[e]);
+      for (uint64_t m = __ballot(live && qrange[e] + crange > LIMIT); m; m &= m - 1) {
+        const int l = __ffsll((long long)m) - 1;
+        float qs[SPAN];
+        load_query_slice<QT, SPAN>(q + ((rt + (l >> 4) + 4 * e) * a.G + g) * D, ln, true, qs);
+        const float c = canonical_score<bf16_t, SPAN>(qs, cent + (int64_t)(tile * 16 + (l & 15)) * D, ln);
+        s = lane == l ? c : s;
+      }
+      if (live) scores[((r - r0) * a.G + g) * a.rows + col] = s;
+    }
+  }
+}
+
+// grid (rows of the slab x G): the K best of a row's visible scores, sorted, and the expansion
+// into its read list, as select_flat_kernel's. Later rows see more buckets: longest first.
+__global__ __launch_bounds__(LSA_BLOCK) void select_scored_kernel(FlatArgs a, int64_t i0, const float* scores) {
+  extern __shared__ uint64_t smem[];
+  __shared__ RadixState st;
+  __shared__ TopkScratch tks;
+  __shared__ BinScratchWide bins;
+  __shared__ int scan[LSA_WAVES];
+  uint64_t* keys = smem;            // [rows]
+  uint64_t* best = smem + a.rows;   // [kp]
+  const int64_t il = gridDim.x - 1 - blockIdx.x;
+  const int64_t i = i0 + il, r = i / a.G, g = i % a.G;
+  const int64_t position = a.positions[r];
+  const int64_t t = g * a.group_tables;
+  const int32_t* ends = a.ends ? a.ends + t * a.rows : nullptr;
+  const int32_t* vends = a.vends ? a.vends + t * a.rows : nullptr;
+  const int vis = vends ? a.rows : max(visible_closed(position, a.rows, a.cluster_block, a.block_buckets), 0);
+  const int n = max(vis, a.K);  // the keys past the visible ones are EMPTY
+  const float* row = scores + il * (int64_t)a.rows;
+  constexpr int U = 8;
+  for (int j0 = 0; j0 < n; j0 += U * LSA_BLOCK) {
+    float s[U];
+    int32_t e[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {  // unconditional (clamped): all in flight
+      const int j = j0 + u * LSA_BLOCK + threadIdx.x;
+      const int jc = j < vis ? j : 0;
+      s[u] = row[jc];
+      e[u] = vends ? vends[jc] : 0;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int j = j0 + u * LSA_BLOCK + threadIdx.x;
+      const bool keep = j < vis && (int64_t)e[u] <= (vends ? position + 1 : 0);
+      if (j < n) keys[j] = keep ? key_to_u(pack_key(s[u], j)) : 0;
+    }
+  }
+  __syncthreads();
+  block_topk_any(keys, n, a.K, a.kp, best, &tks, &st, &bins);
+  int32_t* pk = (int32_t*)keys;
+  for (int j = threadIdx.x; j < a.K; j += LSA_BLOCK) pk[j] = key_column(u_to_key(best[j]));
+  __syncthreads();
+  expand_row(a, pk, t, ends, position, i, scan);
+}
+
+constexpr int64_t kScoreSlabBytes = 128 << 20;  // scores of a slab of rows
+
+// Rows of a slab (a multiple of 16).
+int64_t score_slab_rows(int64_t R, int32_t G, int32_t rows) {
+  const int64_t fit = kScoreSlabBytes / ((int64_t)G * rows * (int64_t)sizeof(float)) / 16 * 16;
+  const int64_t all = (R + 15) / 16 * 16;
+  return fit < 16 ? 16 : (fit < all ? fit : all);
+}
+
+template <typename QT, int D>
+void launch_scored(const QT* q, const FlatArgs& a, size_t shmem, float* scores, hipStream_t s) {
+  const int64_t slab = score_slab_rows(a.R, a.G, a.rows);
+  for (int64_t r0 = 0; r0 < a.R; r0 += slab) {
+    const int64_t r1 = a.R - r0 < slab ? a.R : r0 + slab;
+    const int64_t row_tiles = (r1 - r0 + 15) / 16 * a.G;
+    const int most = (a.rows + 16 * kTileWaves - 1) / (16 * kTileWaves);
+    const int64_t want = (2048 + row_tiles - 1) / row_tiles;  // about eight workgroups a CU
+    const dim3 grid((unsigned)row_tiles, (unsigned)(want < most ? want : most));
+    score_tiles_kernel<QT, D><<<grid, LSA_BLOCK, 0, s>>>(q, a, r0, r1, scores);
+    select_scored_kernel<<<dim3((unsigned)((r1 - r0) * a.G)), LSA_BLOCK, shmem, s>>>(a, r0 * a.G, scores);
+  }
+}
+
 // ------------------------------------------------------------------ two-level tree select
 
 constexpr int kSeenBits = 8192;  // buckets a tree table may hold for the LDS dedup bitmap
@@ -742,14 +928,24 @@ extern "C" size_t lsa_select_flat_scratch_bytes(int64_t R, int32_t G, int32_t to
   return (size_t)(R * G) * (size_t)N * sizeof(uint64_t);
 }
 
-extern "C" int lsa_select_flat(const void* queries, int q_dtype, int64_t R, int32_t G, int32_t D,
-                               const void* centroids, const int32_t* members, const int32_t* ends,
-                               int32_t table_flags, int32_t rows,
-                               int32_t cap, int64_t row_tables, int64_t group_tables, int score_mode,
-                               const int32_t* positions, const lsa_slot_map* slots, int32_t cluster_block_size,
-                               int32_t block_buckets, int32_t top_p, int32_t window, int32_t sink, int32_t top_k,
-                               int32_t splits, int32_t* counters, void* scratch, size_t scratch_bytes,
-                               int32_t* lists, int32_t* lengths, void* stream) {
+// Whether the scores of many rows are made as matrix tiles first: bf16 scores against one table a
+// group.
+extern "C" size_t lsa_select_rows_scratch_bytes(int64_t R, int32_t G, int32_t D, int32_t rows, int32_t top_p,
+                                                int64_t row_tables, int score_mode) {
+  if (R < 1 || G < 1 || rows < 1 || top_p < 1 || row_tables != 0 || score_mode != LSA_SCORE_BF16) return 0;
+  if (!(D == 64 || D == 128) || R * G > 0x7FFFFFFF) return 0;
+  return (size_t)score_slab_rows(R, G, rows) * (size_t)G * (size_t)rows * sizeof(float);
+}
+
+// lsa_select_flat and lsa_select_rows; `tiles`: the scratch holds a slab's scores.
+static int select_flat_impl(const void* queries, int q_dtype, int64_t R, int32_t G, int32_t D,
+                            const void* centroids, const int32_t* members, const int32_t* ends,
+                            int32_t table_flags, int32_t rows,
+                            int32_t cap, int64_t row_tables, int64_t group_tables, int score_mode,
+                            const int32_t* positions, const lsa_slot_map* slots, int32_t cluster_block_size,
+                            int32_t block_buckets, int32_t top_p, int32_t window, int32_t sink, int32_t top_k,
+                            int32_t splits, int32_t* counters, void* scratch, size_t scratch_bytes, bool tiles,
+                            int32_t* lists, int32_t* lengths, void* stream) {
   LSA_REQUIRE(queries && centroids && members && positions && lists && lengths, LSA_ERR_NULL,
               "lsa_select_flat: NULL pointer");
   SlotMap sm;
@@ -777,7 +973,13 @@ extern "C" int lsa_select_flat(const void* queries, int q_dtype, int64_t R, int3
   const int kp = next_pow2(K);
   LSA_REQUIRE(rows + kp <= kMaxLdsKeys, LSA_ERR_SHAPE,
               "lsa_select_flat: %d columns + %d picks exceed %d LDS keys", rows, kp, kMaxLdsKeys);
-  const size_t need = lsa_select_flat_scratch_bytes(R, G, top_p, rows, splits);
+  const size_t need = tiles ? 0 : lsa_select_flat_scratch_bytes(R, G, top_p, rows, splits);
+  const size_t need_rows = tiles ? lsa_select_rows_scratch_bytes(R, G, D, rows, top_p, row_tables, score_mode) : 0;
+  LSA_REQUIRE(!tiles || need_rows > 0, LSA_ERR_SHAPE, "lsa_select_rows: shape not served");
+  LSA_REQUIRE(!tiles || (scratch && ((uintptr_t)scratch & 15) == 0 && scratch_bytes >= need_rows), LSA_ERR_WORKSPACE,
+              "lsa_select_rows: scratch missing, unaligned or %zu < %zu bytes", scratch_bytes, need_rows);
+  LSA_REQUIRE(!tiles || (((uintptr_t)queries | (uintptr_t)centroids) & 15) == 0, LSA_ERR_ALIGN,
+              "lsa_select_rows: queries and centroids must be 16-byte aligned");
   LSA_REQUIRE(need == 0 || (scratch && counters && scratch_bytes >= need), LSA_ERR_WORKSPACE,
               "lsa_select_flat: counters/scratch missing or scratch %zu < %zu bytes", scratch_bytes, need);
   if (R * G == 0) return LSA_OK;
@@ -802,8 +1004,16 @@ extern "C" int lsa_select_flat(const void* queries, int q_dtype, int64_t R, int3
   a.wide_stage = (a.spans && K > LSA_WAVE && width % 4 == 0 && ((uintptr_t)lists % 16) == 0 &&
                   ((4 * (size_t)K + 15) & ~(size_t)15) + stage_lds <= sizeof(uint64_t) * (size_t)rows)
                      ? 1 : 0;
-  a.screen = splits == 1 && score_mode == LSA_SCORE_BF16 && screen_pays(D, rows, K) ? 1 : 0;
+  a.screen = !tiles && splits == 1 && score_mode == LSA_SCORE_BF16 && screen_pays(D, rows, K) ? 1 : 0;
   size_t shmem = base_lds + (a.stage ? stage_lds : 0);
+  if (tiles) {
+    LSA_DISPATCH_QT(q_dtype, {
+      if (D == 128) launch_scored<QT, 128>((const QT*)queries, a, shmem, (float*)scratch, (hipStream_t)stream);
+      else launch_scored<QT, 64>((const QT*)queries, a, shmem, (float*)scratch, (hipStream_t)stream);
+    })
+    LSA_LAUNCHED("lsa_select_rows");
+    return LSA_OK;
+  }
   const size_t screen_lds = sizeof(ScreenLds) + sizeof(uint64_t) * (size_t)kp;
   if (a.screen && screen_lds > shmem) shmem = screen_lds;
   const dim3 grid((unsigned)(R * G), (unsigned)splits);
@@ -815,6 +1025,30 @@ extern "C" int lsa_select_flat(const void* queries, int q_dtype, int64_t R, int3
   }))
   LSA_LAUNCHED("lsa_select_flat");
   return LSA_OK;
+}
+
+extern "C" int lsa_select_flat(const void* queries, int q_dtype, int64_t R, int32_t G, int32_t D,
+                               const void* centroids, const int32_t* members, const int32_t* ends,
+                               int32_t table_flags, int32_t rows,
+                               int32_t cap, int64_t row_tables, int64_t group_tables, int score_mode,
+                               const int32_t* positions, const lsa_slot_map* slots, int32_t cluster_block_size,
+                               int32_t block_buckets, int32_t top_p, int32_t window, int32_t sink, int32_t top_k,
+                               int32_t splits, int32_t* counters, void* scratch, size_t scratch_bytes,
+                               int32_t* lists, int32_t* lengths, void* stream) {
+  return select_flat_impl(queries, q_dtype, R, G, D, centroids, members, ends, table_flags, rows, cap, row_tables,
+                          group_tables, score_mode, positions, slots, cluster_block_size, block_buckets, top_p, window,
+                          sink, top_k, splits, counters, scratch, scratch_bytes, false, lists, lengths, stream);
+}
+
+extern "C" int lsa_select_rows(const void* queries, int q_dtype, int64_t R, int32_t G, int32_t D,
+                               const void* centroids, const int32_t* members, const int32_t* ends,
+                               int32_t table_flags, int32_t rows, int32_t cap, int64_t group_tables, int score_mode,
+                               const int32_t* positions, const lsa_slot_map* slots, int32_t cluster_block_size,
+                               int32_t block_buckets, int32_t top_p, int32_t window, int32_t sink, int32_t top_k,
+                               void* scratch, size_t scratch_bytes, int32_t* lists, int32_t* lengths, void* stream) {
+  return select_flat_impl(queries, q_dtype, R, G, D, centroids, members, ends, table_flags, rows, cap, 0, group_tables,
+                          score_mode, positions, slots, cluster_block_size, block_buckets, top_p, window, sink, top_k,
+                          1, nullptr, scratch, scratch_bytes, true, lists, lengths, stream);
 }
 
 extern "C" int lsa_select_tree(const void* queries, int q_dtype, int64_t R, int32_t G, int32_t D,

@@ -59,6 +59,9 @@ SIGNATURES = {
     "lsa_select_flat_scratch_bytes": (_sz, [_i64, _i32, _i32, _i32, _i32]),
     "lsa_select_flat": (_int, [_p, _int, _i64, _i32, _i32, _p, _p, _p, _i32, _i32, _i32, _i64, _i64, _int, _p, _p, _i32,
                                _i32, _i32, _i32, _i32, _i32, _i32, _p, _p, _sz, _p, _p, _p]),
+    "lsa_select_rows_scratch_bytes": (_sz, [_i64, _i32, _i32, _i32, _i32, _i64, _int]),
+    "lsa_select_rows": (_int, [_p, _int, _i64, _i32, _i32, _p, _p, _p, _i32, _i32, _i32, _i64, _int, _p, _p, _i32, _i32,
+                               _i32, _i32, _i32, _i32, _p, _sz, _p, _p, _p]),
     "lsa_select_tree": (_int, [_p, _int, _i64, _i32, _i32, _p, _p, _i32, _i32, _p, _p, _p, _i32, _i32, _i32, _i64, _i64,
                                _int, _p, _p, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _p, _p, _p]),
     "lsa_select_beam": (_int, [_p, _int, _i64, _i32, _i32, _i32, _p, _p, _p, _i32, _i32, _i32, _p, _p, _p, _i32, _i32,

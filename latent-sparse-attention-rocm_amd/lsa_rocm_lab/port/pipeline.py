@@ -381,6 +381,22 @@ def _select_splits(R: int, G: int, rows: int, top_p: int) -> int:
     return max(1, min(math.ceil(rows / 32), cap, max(1, 2048 // max(units, 1))))
 
 
+# Scores (rows x groups x buckets) from which a select's two launches and fp32 scores in memory
+# cost less than a workgroup a row that scores its table for itself. Both sides, flat select in us
+# as called (general / tiles): 600 rows of 64 buckets 21 / 26, 2048 chunk-groups of 256
+# buckets 46 / 36, 2048 rows of 256 buckets 56 / 44, 4096 chunk-groups of 512 buckets 102 / 72,
+# 32768 rows of 4096 buckets 5180 / 1337; 512 chunk-groups of 512 buckets 26 / 26.
+_ROWS_MIN_SCORES = 1 << 19
+
+
+def _rows_pay(R: int, G: int, rows: int) -> bool:
+    """Whether a flat select of R query rows against one table a group scores them as matrix
+    tiles of 16 rows (``lsa_select_rows``): many rows, and many scores."""
+    if "LSA_SELECT_SPLITS" in os.environ:
+        return False
+    return R >= 64 and R * G >= 256 and R * G * rows >= _ROWS_MIN_SCORES
+
+
 def _decode_splits(dtype, D: int, group: int, units: int, rows: int, top_p: int, score_mode: int,
                    table_flags: int) -> int:
     """Select workgroups per (row, kv-head) of the fused decode: the splits of the rank form
@@ -435,10 +451,23 @@ def _fused_select(index_queries, positions, buckets, config, top_k, score_dtype,
     members = buckets.members.to(device=device, dtype=torch.int32).contiguous()
     ends = _ends(buckets)
     pos = _positions32(positions, device)
-    splits = _select_splits(layout.R, layout.G, layout.rows, config.top_p)
     width = top_k + config.window_size + config.sink_size
     lists = torch.empty(layout.out_shape(width), dtype=torch.int32, device=device)
     lengths = torch.empty(layout.out_shape(), dtype=torch.int32, device=device)
+    if _rows_pay(layout.R, layout.G, layout.rows) and (q.data_ptr() | table.data_ptr()) % 16 == 0:
+        nbytes = _abi.size("lsa_select_rows_scratch_bytes", layout.R, layout.G, layout.D, layout.rows, config.top_p,
+                           layout.row_tables, mode)
+        if nbytes > 0:
+            ws = _abi.Workspace.get(device, "select_rows", nbytes)
+            slots, _keep = _slot_args(slot_table, slot_rows, layout.R, device)
+            _abi.call("lsa_select_rows", q.data_ptr(), _abi.dtype_code(q.dtype), layout.R, layout.G, layout.D,
+                      table.data_ptr(), members.data_ptr(), _abi.ptr(ends), _table_flags(buckets, ends), layout.rows,
+                      members.shape[-1], layout.group_tables, mode, pos.data_ptr(), slots,
+                      config.cluster_block_size, config.block_bucket_count, config.top_p, config.window_size,
+                      config.sink_size, top_k, ws.data_ptr(), nbytes, lists.data_ptr(), lengths.data_ptr(),
+                      _abi.stream(device))
+            return lists, lengths
+    splits = _select_splits(layout.R, layout.G, layout.rows, config.top_p)
     nbytes = _abi.size("lsa_select_flat_scratch_bytes", layout.R, layout.G, config.top_p, layout.rows, splits)
     ws = _abi.Workspace.get(device, "select", nbytes)
     counters = _abi.Counters.get(device, layout.R * layout.G) if nbytes else None
