@@ -10,6 +10,7 @@ no CPU fallback.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 import pathlib
 import threading
@@ -161,6 +162,13 @@ def size(name: str, *args) -> int:
     return int(getattr(load(), name)(*args))
 
 
+@functools.lru_cache(maxsize=4096)
+def shape_size(name: str, *numbers: int) -> int:
+    """``size`` of an entry point that computes from its numbers alone (no pointer, state or
+    device), remembered: a decode step asks for the same shape every time."""
+    return size(name, *numbers)
+
+
 class SlotMap(ctypes.Structure):
     """``lsa_slot_map`` (include/lsa_rocm.h): a paged cache's slot table."""
 
@@ -181,7 +189,8 @@ def ptr(t: torch.Tensor | None) -> int | None:
 
 
 def stream(device: torch.device | None = None) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The current stream's handle (without making a ``torch.cuda.Stream`` of it)."""
+    return torch._C._cuda_getCurrentRawStream(device_index(device))
 
 
 def device_index(device: torch.device | int | str | None) -> int:
@@ -190,7 +199,8 @@ def device_index(device: torch.device | int | str | None) -> int:
         return torch.cuda.current_device()
     if isinstance(device, int):
         return device
-    device = torch.device(device)
+    if not isinstance(device, torch.device):
+        device = torch.device(device)
     return torch.cuda.current_device() if device.index is None else device.index
 
 
@@ -262,12 +272,22 @@ class StatusWord:
     reads without a device sync."""
 
     _words: dict[tuple[int, str], torch.Tensor] = {}
+    _views: dict[tuple[int, str], ctypes.c_int32] = {}  # the same memory, read without a tensor op
 
     @classmethod
     def get(cls, device: torch.device, purpose: str = "decode") -> torch.Tensor:
         key = (device_index(device), purpose)
         word = cls._words.get(key)
-        if word is None:
-            word = torch.zeros(1, dtype=torch.int32, pin_memory=True)
-            cls._words[key] = word
+        if word is None:  # of two threads' words the first kept is the one both use
+            word = cls._words.setdefault(key, torch.zeros(1, dtype=torch.int32, pin_memory=True))
         return word
+
+    @classmethod
+    def check(cls, device: torch.device, purpose: str = "decode") -> tuple[torch.Tensor, int]:
+        """The word and its value now."""
+        word = cls.get(device, purpose)
+        key = (device_index(device), purpose)
+        view = cls._views.get(key)
+        if view is None:  # words are never freed
+            view = cls._views[key] = ctypes.c_int32.from_address(word.data_ptr())
+        return word, view.value

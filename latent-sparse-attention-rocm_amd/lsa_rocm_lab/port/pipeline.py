@@ -136,19 +136,31 @@ def _on_device(what: str, *tensors: torch.Tensor | None) -> torch.device:
     return device
 
 
+def _ready(t: torch.Tensor, dtype: torch.dtype, device: torch.device) -> torch.Tensor:
+    """``t`` as a kernel reads it; nothing is dispatched for a table kept so. A direct decode call is
+    bound by the host: the no-op conversions, the meta tensor, the stream objects and the size
+    queries of one took 10 us (the 2k fp32 step 28.9 -> 18.7 us, the default stages at batch 8
+    95 -> 76)."""
+    if t.dtype == dtype and t.is_contiguous() and t.device == device:
+        return t
+    return t.to(device=device, dtype=dtype).contiguous()
+
+
 class _Layout:
     """How query rows and groups map onto a stack of bucket tables."""
 
-    def __init__(self, index_queries: torch.Tensor, table: torch.Tensor):
-        if index_queries.dim() == 2:
-            self.R, self.D = index_queries.shape
+    def __init__(self, index_queries: torch.Tensor | tuple[int, ...], table: torch.Tensor):
+        """``index_queries``: the tensor, or its shape where a kernel makes it."""
+        shape = index_queries if isinstance(index_queries, tuple) else tuple(index_queries.shape)
+        if len(shape) == 2:
+            self.R, self.D = shape
             self.G = 1
             self.grouped = False
-        elif index_queries.dim() == 3:
-            self.R, self.G, self.D = index_queries.shape
+        elif len(shape) == 3:
+            self.R, self.G, self.D = shape
             self.grouped = True
         else:
-            raise ValueError(f"index queries must be [R, d] or [R, G, D], got {tuple(index_queries.shape)}")
+            raise ValueError(f"index queries must be [R, d] or [R, G, D], got {shape}")
         lead = table.dim() - 2
         if lead == 0:
             self.row_tables, self.group_tables = 0, 0
@@ -169,22 +181,21 @@ class _Layout:
 
 
 def _positions32(positions: torch.Tensor, device) -> torch.Tensor:
-    p = positions.to(device=device)
-    return (p if p.dtype == torch.int32 else p.to(torch.int32)).contiguous()
+    return _ready(positions, torch.int32, device)
 
 
 def _score_table(buckets: Buckets, score_dtype: str) -> tuple[torch.Tensor, int]:
     if score_dtype == "fp32":
         if buckets.centroids_f32 is None:
             raise ValueError("fp32 scoring needs buckets.centroids_f32")
-        return buckets.centroids_f32.float().contiguous(), _abi.SCORE_F32
+        return _ready(buckets.centroids_f32, torch.float32, buckets.centroids_f32.device), _abi.SCORE_F32
     if score_dtype != "bf16":
         raise ValueError(f"score_dtype must be bf16|fp32, got {score_dtype!r}")
-    return buckets.centroids.to(torch.bfloat16).contiguous(), _abi.SCORE_BF16
+    return _ready(buckets.centroids, torch.bfloat16, buckets.centroids.device), _abi.SCORE_BF16
 
 
 def _ends(buckets: Buckets) -> torch.Tensor | None:
-    return None if buckets.ends is None else buckets.ends.to(torch.int32).contiguous()
+    return None if buckets.ends is None else _ready(buckets.ends, torch.int32, buckets.ends.device)
 
 
 def _table_flags(buckets: Buckets, ends: torch.Tensor | None) -> int:
@@ -328,7 +339,7 @@ def _expand(picks: torch.Tensor, picks_are_keys: bool, layout: _Layout, members:
             positions: torch.Tensor, window: int, sink: int, top_k: int, slot_table=None, slot_rows=None):
     device = picks.device
     picks = picks.contiguous()
-    members = members.to(device=device, dtype=torch.int32).contiguous()
+    members = _ready(members, torch.int32, device)
     P = picks.shape[-1]
     width = top_k + window + sink
     lists = torch.empty(layout.out_shape(width), dtype=torch.int32, device=device)
@@ -409,8 +420,8 @@ def _decode_splits(dtype, D: int, group: int, units: int, rows: int, top_p: int,
     mode = os.environ.get("LSA_DECODE_MODE", "auto")
     if mode not in ("auto", "rep", "exchange"):
         raise ValueError(f"LSA_DECODE_MODE must be auto|rep|exchange, got {mode!r}")
-    ok = bool(_abi.load().lsa_decode_flat_rep_ok(_abi.dtype_code(dtype), D, group, rows, top_p, score_mode,
-                                                 table_flags))
+    ok = bool(_abi.shape_size("lsa_decode_flat_rep_ok", _abi.dtype_code(dtype), D, group, rows, top_p, score_mode,
+                              table_flags))
     if mode == "rep" and not ok:
         raise ValueError("LSA_DECODE_MODE=rep: the replicated select does not apply to this shape")
     if ok and (mode == "rep" or (mode == "auto" and units <= _REP_MAX_UNITS)):
@@ -448,7 +459,7 @@ def _fused_select(index_queries, positions, buckets, config, top_k, score_dtype,
     layout = _Layout(index_queries, buckets.centroids)
     table, mode = _score_table(buckets, score_dtype)
     q = _queries(index_queries)
-    members = buckets.members.to(device=device, dtype=torch.int32).contiguous()
+    members = _ready(buckets.members, torch.int32, device)
     ends = _ends(buckets)
     pos = _positions32(positions, device)
     width = top_k + config.window_size + config.sink_size
@@ -468,7 +479,7 @@ def _fused_select(index_queries, positions, buckets, config, top_k, score_dtype,
                       _abi.stream(device))
             return lists, lengths
     splits = _select_splits(layout.R, layout.G, layout.rows, config.top_p)
-    nbytes = _abi.size("lsa_select_flat_scratch_bytes", layout.R, layout.G, config.top_p, layout.rows, splits)
+    nbytes = _abi.shape_size("lsa_select_flat_scratch_bytes", layout.R, layout.G, config.top_p, layout.rows, splits)
     ws = _abi.Workspace.get(device, "select", nbytes)
     counters = _abi.Counters.get(device, layout.R * layout.G) if nbytes else None
     slots, _keep = _slot_args(slot_table, slot_rows, layout.R, device)
@@ -634,9 +645,9 @@ def flat_decode(
     k, v, sb, st, sh = _kv_layout(k, v)
     if k.shape[0] != B:  # one pool read by every batch row
         sb = 0
-    layout = _Layout(torch.empty((B, Hkv, D), device="meta"), buckets.centroids)
+    layout = _Layout((B, Hkv, D), buckets.centroids)
     table, mode = _score_table(buckets, score_dtype)
-    members = buckets.members.to(device=device, dtype=torch.int32).contiguous()
+    members = _ready(buckets.members, torch.int32, device)
     ends = _ends(buckets)
     flags = _table_flags(buckets, ends)
     pos = _positions32(positions, device)
@@ -653,12 +664,12 @@ def flat_decode(
     out = torch.empty_like(q)
     dt = _abi.dtype_code(q.dtype)
     readers = int(os.environ.get("LSA_DECODE_READERS", "0")) if readers is None else readers
-    n_counters = _abi.size("lsa_decode_flat_counters", B, Hkv, rows, config.top_p)
-    nbytes = _abi.size("lsa_decode_flat_scratch_bytes", dt, B, Hq, Hkv, D, rows, config.top_p,
-                       config.window_size, config.sink_size, splits, readers)
+    n_counters = _abi.shape_size("lsa_decode_flat_counters", B, Hkv, rows, config.top_p)
+    nbytes = _abi.shape_size("lsa_decode_flat_scratch_bytes", dt, B, Hq, Hkv, D, rows, config.top_p,
+                             config.window_size, config.sink_size, splits, readers)
     if status is None:
-        status = _abi.StatusWord.get(device)
-        if int(status[0]) != 0:
+        status, gave_up = _abi.StatusWord.check(device)
+        if gave_up:
             _decode_gave_up(device, status)
     ws = _abi.Workspace.get(device, "decode", nbytes)
     counters = _abi.Counters.get(device, max(n_counters, 1))
@@ -749,11 +760,11 @@ def flat_decode_shared(
     dt = _abi.dtype_code(q.dtype)
     readers = int(os.environ.get("LSA_DECODE_READERS", "0")) if readers is None else readers
     splits = int(os.environ.get("LSA_SELECT_SPLITS", "0")) if splits is None else splits
-    n_counters = _abi.size("lsa_decode_shared_counters", B, Hkv, rows)
-    nbytes = _abi.size("lsa_decode_shared_scratch_bytes", dt, B, Hq, Hkv, D, rows, config.top_p, config.window_size,
-                       config.sink_size, top_k, readers)
-    status = _abi.StatusWord.get(device)
-    if int(status[0]) != 0:
+    n_counters = _abi.shape_size("lsa_decode_shared_counters", B, Hkv, rows)
+    nbytes = _abi.shape_size("lsa_decode_shared_scratch_bytes", dt, B, Hq, Hkv, D, rows, config.top_p,
+                             config.window_size, config.sink_size, top_k, readers)
+    status, gave_up = _abi.StatusWord.check(device)
+    if gave_up:
         _decode_gave_up(device, status)
     ws = _abi.Workspace.get(device, "decode_shared", nbytes)
     counters = _abi.Counters.get(device, max(n_counters, 1))
@@ -872,10 +883,10 @@ def tree_decode_shared(
     n_nodes = (ctypes.c_int32 * n_levels)(*[kk.shape[-2] for kk in kids])
     levels = min(n_levels, config.top_level)
     n_counters = _abi.size("lsa_decode_tree_shared_counters", B, Hkv, levels, ctypes.addressof(n_nodes), rows)
-    nbytes = _abi.size("lsa_decode_shared_scratch_bytes", dt, B, Hq, Hkv, D, rows, config.top_p, config.window_size,
-                       config.sink_size, top_k, readers)
-    status = _abi.StatusWord.get(device)
-    if int(status[0]) != 0:
+    nbytes = _abi.shape_size("lsa_decode_shared_scratch_bytes", dt, B, Hq, Hkv, D, rows, config.top_p,
+                             config.window_size, config.sink_size, top_k, readers)
+    status, gave_up = _abi.StatusWord.check(device)
+    if gave_up:
         _decode_gave_up(device, status)
     ws = _abi.Workspace.get(device, "decode_shared", nbytes)
     counters = _abi.Counters.get(device, max(n_counters, 1))
@@ -934,8 +945,8 @@ def tree_decode(
     k, v, sb, st, sh = _kv_layout(k, v)
     if k.shape[0] != B:  # one pool read by every batch row
         sb = 0
-    layout = _Layout(torch.empty((B, Hkv, D), device="meta"), buckets.centroids)
-    node_layout = _Layout(torch.empty((B, Hkv, D), device="meta"), level.centroids)
+    layout = _Layout((B, Hkv, D), buckets.centroids)
+    node_layout = _Layout((B, Hkv, D), level.centroids)
     if (node_layout.row_tables, node_layout.group_tables) != (layout.row_tables, layout.group_tables):
         raise ValueError("node and bucket tables must share the same leading axes")
     table, mode = _score_table(buckets, score_dtype)
@@ -945,7 +956,7 @@ def tree_decode(
         ncent = level.centroids.float()
     ncent = ncent.contiguous()
     children = level.children.to(device=device, dtype=torch.int32).contiguous()
-    members = buckets.members.to(device=device, dtype=torch.int32).contiguous()
+    members = _ready(buckets.members, torch.int32, device)
     ends = _ends(buckets)
     flags = _table_flags(buckets, ends)
     pos = _positions32(positions, device)
@@ -960,11 +971,11 @@ def tree_decode(
     out = torch.empty_like(q)
     dt = _abi.dtype_code(q.dtype)
     readers = int(os.environ.get("LSA_DECODE_READERS", "0")) if readers is None else readers
-    n_counters = _abi.size("lsa_decode_flat_counters", B, Hkv, rows, config.top_p)
-    nbytes = _abi.size("lsa_decode_flat_scratch_bytes", dt, B, Hq, Hkv, D, rows, config.top_p,
-                       config.window_size, config.sink_size, 1, readers)
-    status = _abi.StatusWord.get(device)
-    if int(status[0]) != 0:
+    n_counters = _abi.shape_size("lsa_decode_flat_counters", B, Hkv, rows, config.top_p)
+    nbytes = _abi.shape_size("lsa_decode_flat_scratch_bytes", dt, B, Hq, Hkv, D, rows, config.top_p,
+                             config.window_size, config.sink_size, 1, readers)
+    status, gave_up = _abi.StatusWord.check(device)
+    if gave_up:
         _decode_gave_up(device, status)
     ws = _abi.Workspace.get(device, "decode", nbytes)
     counters = _abi.Counters.get(device, max(n_counters, 1))
@@ -998,8 +1009,8 @@ def check_decode(device: torch.device | int | None = None) -> None:
     fused decode launch on it gave up waiting since the last check."""
     device = torch.device("cuda", _abi.device_index(device))
     torch.cuda.synchronize(device)
-    status = _abi.StatusWord.get(device)
-    if int(status[0]) != 0:
+    status, gave_up = _abi.StatusWord.check(device)
+    if gave_up:
         _decode_gave_up(device, status)
 
 

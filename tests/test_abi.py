@@ -256,3 +256,20 @@ def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setattr(_abi, "LIB_PATH", tmp_path / "absent.so")
     with pytest.raises(_abi.ExtensionMissing):
         _abi.load()
+
+
+@pytest.mark.parametrize("dtype,step", [(torch.int32, 1), (torch.int64, 1), (torch.int32, 2)])
+def test_ready_converts_what_a_kernel_cannot_read(dtype, step):
+    from lsa_rocm_lab.port import pipeline
+
+    t = torch.arange(24, dtype=dtype)[::step]
+    got = pipeline._ready(t, torch.int32, t.device)
+    assert got.dtype == torch.int32 and got.is_contiguous() and torch.equal(got.long(), t.long())
+    assert (got is t) == (dtype == torch.int32 and step == 1)
+
+
+def test_shape_size_is_the_librarys_answer():
+    args = (1, 8, 32, 512, 8)
+    for _ in range(2):
+        assert _abi.shape_size("lsa_select_flat_scratch_bytes", *args) == 8 * 512 * 8
+    assert _abi.shape_size("lsa_select_flat_scratch_bytes", 1, 8, 32, 512, 1) == 0
