@@ -7,6 +7,7 @@ import pathlib
 import re
 
 import pytest
+import torch
 
 from lsa_rocm_lab import _abi
 
