@@ -1,5 +1,6 @@
 """The flat select of many rows (scores as fp64 matrix tiles) against the general fused select,
-a workgroup a row: lists and lengths bit-exact at tile, slab and exponent-range edges."""
+a workgroup a row: lists and lengths bit-exact at tile, slab and exponent-range edges. And the default chain's pick
+counts against the chain that packs and lists its keys."""
 
 import pytest
 import torch
@@ -95,3 +96,20 @@ def test_rows_select_more_rows_than_a_slab(monkeypatch):
     q = torch.randn(8213, 64, device=DEV, generator=gen)
     pos = torch.arange(8213, device=DEV, dtype=torch.int32) * 3
     _both(monkeypatch, q, pos, table, _config(100))
+
+
+@pytest.mark.parametrize("G", [0, 3])
+@pytest.mark.parametrize("rows,top_p", [(1, 1), (200, 1), (200, 33), (33, 64), (300, 257), (5000, 64), (1200, 4096)])
+def test_default_chain_equals_the_listing(monkeypatch, G, rows, top_p):
+    print(f"case chain G={G} rows={rows} top_p={top_p}", flush=True)
+    gen = torch.Generator(device=DEV).manual_seed(rows + top_p)
+    table = _table(G, rows, 64, gen, False)
+    R = 21
+    q = torch.randn(*((R, G) if G else (R,)), 64, device=DEV, generator=gen)
+    q[3] = float("nan")
+    pos = torch.randint(-1, 5 * rows + 64, (R,), device=DEV, generator=gen).to(torch.int32)
+    got = pipeline.flat_select_reference(q, pos, table, _config(top_p))
+    monkeypatch.setenv("LSA_SELECT_IMPL", "fused_unpack")
+    want = pipeline.flat_select(q, pos, table, _config(top_p))
+    torch.cuda.synchronize()
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
