@@ -52,7 +52,8 @@ __host__ __device__ inline bool screen_fits(int D, int rows, int K) {
 // trip of centroid loads (256 rows of 16-bit operands in flight a workgroup), while the
 // screen takes two (the rows, then the candidates' re-score). Measured on the tree
 // decode's selects (128 nodes, then <= 256 candidates): 20.5 us exact vs 22.8 us
-// screened; on the 32k prefill select's 512-row tables the screen wins (102 vs 123 us).
+// screened; on 4096 rows of 512-row tables the screen wins (102 vs 123 us; against one table a
+// group such a call takes lsa_select_rows, 72 us).
 constexpr int kScreenMinRows = 256;
 __host__ __device__ inline bool screen_pays(int D, int rows, int K) {
   return rows > kScreenMinRows && screen_fits(D, rows, K);

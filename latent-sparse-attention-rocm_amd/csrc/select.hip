@@ -192,9 +192,9 @@ __device__ __forceinline__ void expand_row(const FlatArgs& a, const int32_t* pk,
 // publishes the keys and the last split to arrive takes every column's key from the
 // workspace. That workgroup selects the K best keys, sorted, and expands the picks into
 // the read list in rank order (reference pipeline.py:248-316, select_fused.py:52-280).
-// Four waves a SIMD (128 VGPRs, a few spilled): with one workgroup per row, the prefill's
-// 4096 rows are latency-bound and the fourth resident workgroup a CU hides more of it
-// (0.22 -> 0.20 ms for the 32k prefill select; the 8-row decode select is unchanged).
+// Four waves a SIMD (128 VGPRs, a few spilled): with one workgroup per row, a select of
+// thousands of rows is latency-bound and the fourth resident workgroup a CU hides more of it
+// (0.22 -> 0.20 ms for 4096 rows of 512 buckets; the 8-row decode select is unchanged).
 template <typename QT, typename CT, int SPAN>
 __global__ __launch_bounds__(LSA_BLOCK) __attribute__((amdgpu_waves_per_eu(4, 4))) void select_flat_kernel(
     const QT* q, bool bf16_mode, FlatArgs a) {

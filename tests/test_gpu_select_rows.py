@@ -113,3 +113,38 @@ def test_default_chain_equals_the_listing(monkeypatch, G, rows, top_p):
     want = pipeline.flat_select(q, pos, table, _config(top_p))
     torch.cuda.synchronize()
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+def test_rows_select_and_read_in_a_captured_graph():
+    """The many-row select and read as a replayed graph, over new inputs, with eager work between."""
+    gen = torch.Generator(device=DEV).manual_seed(9)
+    R, rows, Hq, Hkv, D = 2048, 300, 8, 2, 64
+    table, config = _table(0, rows, D, gen, False), _config(64)
+    idx = torch.randn(R, D, device=DEV, generator=gen)
+    q, k, v = (torch.randn(1, n, h, D, device=DEV, generator=gen).to(torch.bfloat16)
+               for n, h in ((R, Hq), (3000, Hkv), (3000, Hkv)))
+    pos = torch.arange(R, device=DEV, dtype=torch.int32)
+    assert pipeline._rows_pay(R, 1, rows)
+
+    def step():
+        lists, lengths = pipeline._fused_select(idx, pos, table, config, config.top_k, "bf16")
+        return pipeline.lsa_read(q, k, v, lists[None], lengths[None], D ** -0.5), lists, lengths
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step()
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        out = step()
+    for _ in range(3):
+        idx.copy_(torch.randn(R, D, device=DEV, generator=gen))
+        q.copy_(torch.randn(1, R, Hq, D, device=DEV, generator=gen))
+        want = [t.clone() for t in step()]
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        for got, w in zip(out, want):
+            assert torch.equal(got, w)
