@@ -246,8 +246,9 @@ int lsa_read(const void* q, const void* k, const void* v, int dtype, int64_t B, 
 /* The same read for many query rows over one cache (the reference's prefill: every row has
  * its own list), as a masked sweep on the matrix cores: 256 query columns (rows times the
  * kv-head's query group) a workgroup cross the 64-key tiles any of their rows lists, each
- * row's list a bitmap that masks its weights (16-bit halves that add up to the fp32 weight
- * within 2^-17). Rows the sweep does not serve - a list naming a key twice, a tile whose K or V
+ * row's list a bitmap that masks its weights (two 16-bit halves that add up to the fp32 weight
+ * within 2^-17 of it in bf16, and in fp16 within 2^-23 of it or 2^-37 of the row's largest weight,
+ * whichever is more). Rows the sweep does not serve - a list naming a key twice, a tile whose K or V
  * is not finite, too few listed keys for the tiles crossed - are read by the gather in the
  * same call. Arguments as lsa_read's; bf16/fp16 rows of head dim 64 or 128, at most 262144
  * cache rows, kv_token_stride below 2^24, scale > 0. lsa_read_rows_scratch_bytes(): 0 where it

@@ -35,7 +35,6 @@ constexpr int NB = 4;                  // K and V tile buffers each
 constexpr int kBlockRows = 32;         // query rows of a bitmap block (and columns of a wave)
 constexpr int kMaxTiles = 4096;        // tiles of a cache (262144 rows)
 constexpr int64_t kSlabBytes = 64 << 20;
-constexpr float kGrow = 8.0f;          // log2 growth of a column maximum that forces a rescale
 
 struct RowsArgs {
   const void* q;
@@ -268,8 +267,14 @@ __device__ __forceinline__ uint32_t bit_mask(uint32_t w, int bit) {
 
 // A wave's 32 query columns: LDS addresses, the matrix products, and the weights of a tile. The
 // gather read multiplies fp32 weights, so here a weight enters the matrix cores as the sum of
-// two 16-bit halves, within 2^-17 of it (one half alone would cost 2^-9); the normaliser adds
-// up the fp32 weights.
+// two 16-bit halves (one alone would cost 2^-9 of it); the normaliser adds up the fp32 weights.
+// bf16 halves are within 2^-17 of the weight at any size (fp32's exponents). fp16 halves are
+// within 2^-23, but end at 2^-24: weights below that would count in the normaliser alone, and
+// rows of one large and many small weights lost all the small ones (4612 keys of 2^-25 beside one of
+// 1 read 0 for 1.4e-4). So fp16 weights are kept as high as their range allows: the largest is 2^BIAS
+// when the reference moves and stays below 2^TOP, and the smallest step of a half is 2^-36 of it
+// (8192 rows of 4612 keys, 32 heads on 8: D 128 827 -> 860 us, D 64 590 -> 629). Measured against
+// 64 bits, 4096 rows of up to 2308 keys: 2.1e-4 in fp16 and 1.7e-3 in bf16, as the gather.
 template <typename T, int D>
 struct Sweep {
   using M = Mfma<T>;
@@ -277,6 +282,9 @@ struct Sweep {
   static constexpr int KS = D / 16, DB = D / 32, SEGS = D / 8, ROWB = 2 * D;
   static constexpr int KPI = 1024 / ROWB;            // keys a dma16 moves
   static constexpr int NI = kTile / (KPI * kWaves);  // dma16s a wave a tile, K and V each
+  // log2 of a column's largest weight when its reference moves, and of the weight that moves it
+  static constexpr bool HALF = !__is_same(T, bf16_t);
+  static constexpr float BIAS = HALF ? 12.0f : 0.0f, TOP = HALF ? 15.0f : 8.0f;
 
   const lds_char *kl, *vl;
   uint32_t kbase, vbase;
@@ -284,7 +292,7 @@ struct Sweep {
   op_t qop[KS];
   f32x16_t o[DB], sc[2];
   uint32_t ph[2][8], pl[2][8];  // the weights' halves, two a word
-  float m_run, l_run;
+  float m_run, l_run;  // the weights' reference, 2^BIAS below the largest score when it moved; their sum
   Rest<T> rest;
 
   __device__ __forceinline__ void init(const void* k_tiles, const void* v_tiles, const T* qrow) {
@@ -397,9 +405,13 @@ struct Sweep {
   // them after the other: one wave a SIMD makes weights, so a chain of dependent instructions
   // would leave the unit idle between them (16k rows: 3.15 ms with four at a time, 2.98 with
   // eight, 3.00 with sixteen).
-  __device__ __forceinline__ void weights(const uint32_t (&wd)[2], float scale_log2, float (&ls)[2]) {
+  // top: the largest upper halves of even and odd keys, as bits (weights are not negative, so the
+  // bits order as they do); fp16.
+  typedef unsigned short u16x2_t __attribute__((ext_vector_type(2)));
+  __device__ __forceinline__ void weights(const uint32_t (&wd)[2], float scale_log2, float (&ls)[2], u16x2_t& top) {
     constexpr int E = 8;
     ls[0] = ls[1] = 0.0f;
+    top = {0, 0};
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
 #pragma unroll
@@ -423,6 +435,10 @@ struct Sweep {
         for (int e = 0; e < E; e += 2) pair[e / 2] = M::pack2(p[e], p[e + 1]);
 #pragma unroll
         for (int e = 0; e < E; ++e) ls[e & 1] += p[e];
+        if constexpr (HALF) {
+#pragma unroll
+          for (int e = 0; e < E / 2; ++e) top = __builtin_elementwise_max(top, __builtin_bit_cast(u16x2_t, pair[e]));
+        }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int e = 0; e < E; e += 2) {
@@ -436,18 +452,20 @@ struct Sweep {
       }
     }
   }
-  // The weights of a tile and its share of the normaliser. The running maximum moves lazily:
-  // the weights are made against the current one, and only where a lane's 32 weights reach
-  // 2^kGrow (or are not numbers) are the column maxima taken and, where a column grew by more
-  // than 2^kGrow, the state rescaled and the weights made again. So every weight stays below
-  // 2^kGrow, and most tiles take no maximum.
+  // The weights of a tile and its share of the normaliser. The reference moves lazily: the weights
+  // are made against the current one, and only where a weight may have reached 2^TOP (bf16: a
+  // lane's 32 weights together, which costs no instruction; fp16, whose range leaves no room for
+  // that, the largest one) are the column maxima taken and, where a column's did, the state
+  // rescaled and the weights made again. So every weight stays below 2^TOP, and most tiles take
+  // no maximum.
   __device__ __forceinline__ void softmax(uint64_t mask, float scale_log2) {
     const int hh = (threadIdx.x & 63) / 32;
     const uint32_t wd[2] = {(uint32_t)mask >> (4 * hh), (uint32_t)(mask >> 32) >> (4 * hh)};
     float ls[2];
-    weights(wd, scale_log2, ls);
-    static_assert(kGrow == 8.0f, "the sum test is against 2^kGrow");
-    if (__any(!(ls[0] + ls[1] < 256.0f))) {
+    u16x2_t top;
+    weights(wd, scale_log2, ls, top);
+    static_assert(TOP == (HALF ? 15.0f : 8.0f), "the test is against 2^TOP");
+    if (__any(HALF ? max(top.x, top.y) >= 0x7800 : !(ls[0] + ls[1] < 256.0f))) {
       float mx = -INFINITY;
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
@@ -455,8 +473,8 @@ struct Sweep {
         for (int r = 0; r < 16; ++r) mx = fmaxf(mx, (wd[h] >> (8 * (r / 4) + r % 4)) & 1u ? sc[h][r] : -INFINITY);
       }
       const float mt = fmaxf(mx, lane_xor(mx, 32)) * scale_log2;
-      if (__any(mt > m_run + kGrow)) {
-        const float mn = fmaxf(m_run, mt);
+      if (__any(mt > m_run + TOP)) {
+        const float mn = fmaxf(m_run, mt - BIAS);
         const float alpha = fast_exp2(m_run - mn);
         m_run = mn;
         l_run *= alpha;
@@ -465,7 +483,7 @@ struct Sweep {
 #pragma unroll
           for (int r = 0; r < 16; ++r) o[d][r] *= alpha;
         }
-        weights(wd, scale_log2, ls);
+        weights(wd, scale_log2, ls, top);
       }
     }
     l_run += ls[0] + ls[1];

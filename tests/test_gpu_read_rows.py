@@ -132,6 +132,34 @@ def test_large_scores():
     check(q * 6, k * 4, v, ids, lengths)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n", [4611, 40000])
+def test_small_weights_beside_a_large_one(dtype, n):
+    """A row of one key of weight 1 (V 0) and n of weight 2^-x (V 1): what is read is the small
+    ones' share, about n 2^-x.
+
+    Bound: the output's rounding (its smallest step in fp16 2^-24); 2^-9 of the share for bf16's
+    split weights, the exponent's rounding (x 2^-24 of it) and fp32 sums of n / 8 terms; and in
+    fp16 2^-37 a weight."""
+    D, half = 64, dtype == torch.float16
+    q = torch.zeros(1, 64, 4, D, dtype=dtype)
+    q[..., 0] = 1
+    k = torch.zeros(1, n + 1, 1, D, dtype=dtype)
+    v = torch.ones(1, n + 1, 1, D, dtype=dtype)
+    v[0, 0] = 0
+    ids = torch.arange(n + 1, dtype=torch.int32).expand(1, 64, n + 1).contiguous()
+    lengths = torch.full((1, 64), n + 1, dtype=torch.int32)
+    scale = float(np.float32(np.log(2.0)))
+    for x in (8, 16, 20, 23.5, 24.5, 25.25, 27.25, 30.25, 33, 36):
+        k[0, :, 0, 0], k[0, 0, 0, 0] = -x / 2, x / 2  # exact in both types
+        w = np.exp(-x * scale)
+        want = n * w / (1 + n * w)
+        got = sweep(q, k, v, ids, lengths, scale=scale).double().cpu().numpy()
+        bound = (RTOL[dtype] + 2.0 ** -9) * want + (n * 2.0 ** -37 + 2.0 ** -25 if half else 0.0)
+        err = np.abs(got - want).max()
+        assert err <= bound, (x, got.flat[0], want, err, bound)
+
+
 def test_segments_and_slabs():
     """A 262144-row cache (eight bitmap segments, a slab of 64 row tiles) under 2080 rows: both
     slabs' rows against the oracle, keys of every segment."""
