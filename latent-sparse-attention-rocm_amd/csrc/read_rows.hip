@@ -7,17 +7,17 @@
 // sweep the 64-key tiles any of their rows lists, and each row's list, as a bitmap over the
 // cache rows, masks the softmax weights: the keys outside it weigh exactly zero.
 //
-//   tile_finite_kernel  flags the 64-key tiles whose K or V holds a value that is not finite
-//                       (a masked product would not be zero there);
 //   row_bits_kernel     turns 32 rows' lists into bitmaps (bits [block][tile][row], 64 bits
 //                       each) and flags, per block and tile, whether any row lists a key there,
 //                       and the rows that list a key twice (a bitmap cannot count);
+//   tile_finite_kernel  flags the 64-key tiles whose K or V holds a value that is not finite
+//                       (a masked product would not be zero there);
 //   rows_mfma_kernel    the sweep, 256 columns a workgroup;
 //   rows_rest_kernel    the gather read of the rows the sweep leaves out: a duplicate in the
 //                       list, a flagged tile among the workgroup's, or too few listed keys for
 //                       the tiles they are spread over.
 //
-// A slab of query rows at a time, so that the bitmaps stay under kSlabBytes.
+// A slab of query rows at a time, so that the bitmaps (and the list of units left) stay under kSlabBytes.
 #include <math.h>
 
 #include "lsa_abi_common.h"
@@ -35,6 +35,8 @@ constexpr int NB = 4;                  // K and V tile buffers each
 constexpr int kBlockRows = 32;         // query rows of a bitmap block (and columns of a wave)
 constexpr int kMaxTiles = 4096;        // tiles of a cache (262144 rows)
 constexpr int64_t kSlabBytes = 64 << 20;
+constexpr int kXcds = 8;
+constexpr int64_t kRestGrid = 16384;   // most workgroups that gather what is left (a multiple of kXcds)
 
 struct RowsArgs {
   const void* q;
@@ -55,8 +57,11 @@ struct RowsArgs {
   uint64_t* bits;      // [block][tile][32 rows]
   uint8_t* any;        // [block][tile]
   uint8_t* dup;        // [block][32 rows]
-  uint8_t* rest;       // [row tile][kv-head]: 1 the sweep leaves the tile to the gather
-  const uint8_t* odd;  // [batch of K][kv-head][tile]: a value that is not finite
+  int2* listed;        // [block]: keys its rows list (rows without duplicates), tiles they lie in
+  int* left_n;         // [kXcds]: units (row, kv-head) of the slab left to the gather, by list
+  int32_t* left;       // [kXcds][left_cap]: them, (row of the slab's row tiles) * kv-heads + kv-head
+  int left_cap;
+  const uint8_t* odd;  // [batch of K][kv-head][tile]: 1 a value that is not finite, or kUnseen
   float scale_log2;
   int empty_nan;
 };
@@ -66,6 +71,67 @@ __device__ __forceinline__ int64_t list_of(const RowsArgs& a, int64_t b, int64_t
   const int64_t row = b * a.Tq + t;
   return a.per_head ? row * a.Hkv + g : row;
 }
+
+// ---------------------------------------------------------------- what is swept
+
+// Listed keys a swept tile under which the gather reads a workgroup's rows faster: the sweep
+// takes a CU ~2.6 us a tile (D 64: 1.9), the gather ~7.9 ns a listed key (D 64: 2.7, 3.8, 5.9
+// and 12.3 ns at query groups 1, 2, 4 and 8).
+template <int D, int GQ>
+__device__ constexpr int sparse_keys() {
+  return D == 128 ? 330 : (GQ == 1 ? 700 : (GQ == 2 ? 500 : (GQ == 4 ? 320 : 155)));
+}
+
+// Whether the sweep serves any row of the slab. The host chose it by sizes; the lists may still be
+// short or scattered. A workgroup whose rows list enough keys a tile is swept, but the sweep takes
+// at least its longest workgroup, so a slab of which only some are is read by the gather altogether where
+// that is faster: 2048 rows of 0 to 4612 keys over 32768, 32 heads on 8, D 128, one workgroup in
+// seven dense enough: 2.78 ms, 1.47 by this rule, 1.40 by the gather alone. Every workgroup of a
+// kernel that asks finds the same; of more than 256 lists it looks at evenly spaced ones (an odd step,
+// so that they are not all of one kv-head). Every thread calls both parts, a barrier between them.
+enum Verdict { kGather, kSweep, kNothing };  // kNothing: no keys but duplicates' are listed
+template <int D, int GQ, int THREADS>
+struct SlabVerdict {
+  static constexpr int RB = kWaves / GQ, WAVES = THREADS / LSA_WAVE;
+  typedef float Red[WAVES][4];
+  int keys = 0, tiles = 0, step;
+
+  __device__ __forceinline__ explicit SlabVerdict(const RowsArgs& a) {
+    const int units = a.n_u * (a.per_head ? a.Hkv : 1);
+    step = units <= LSA_BLOCK ? 1 : (units / LSA_BLOCK + 1) | 1;
+    const int64_t i = (int64_t)threadIdx.x * step;
+    if (threadIdx.x < LSA_BLOCK && i < units) {
+#pragma unroll
+      for (int r = 0; r < RB; ++r) {
+        const int2 x = a.listed[i * RB + r];
+        keys += x.x;
+        tiles = max(tiles, x.y);  // at least these
+      }
+    }
+  }
+  __device__ __forceinline__ void add_up(Red& red) const {
+    const bool ok = (float)keys >= (float)tiles * (float)sparse_keys<D, GQ>();
+    const float dense = wave_sum(ok ? (float)keys : 0.0f), thin = wave_sum(ok ? 0.0f : (float)keys);
+    const float t = wave_sum(ok ? (float)tiles : 0.0f), longest = wave_max(ok ? (float)tiles : 0.0f);
+    if (threadIdx.x % LSA_WAVE == 0) {
+      float* x = red[threadIdx.x / LSA_WAVE];
+      x[0] = dense; x[1] = thin; x[2] = t; x[3] = longest;
+    }
+  }
+  __device__ __forceinline__ Verdict verdict(const RowsArgs& a, const Red& red) const {
+    constexpr float SPARSE = (float)sparse_keys<D, GQ>(), CUS = 256.0f;
+    float dense = 0.0f, thin = 0.0f, t = 0.0f, longest = 0.0f;
+#pragma unroll
+    for (int x = 0; x < WAVES; ++x) {
+      dense += red[x][0]; thin += red[x][1]; t += red[x][2];
+      longest = fmaxf(longest, red[x][3]);
+    }
+    if (dense + thin == 0.0f) return kNothing;
+    const float all = (a.per_head ? 1.0f : (float)a.Hkv) * (float)step;  // workgroups a list seen
+    const bool pays = 3.0f * thin <= dense || (dense > 0.0f && all * dense >= SPARSE * fmaxf(all * t, CUS * longest));
+    return pays ? kSweep : kGather;
+  }
+};
 
 // ---------------------------------------------------------------- tiles that are not finite
 
@@ -79,12 +145,24 @@ __device__ __forceinline__ bool odd16(const uint4& x) {  // any of 8 elements in
   return bad;
 }
 
-// grid (tile, kv-head, batch of K). HBM-bound: one read of K and V.
-template <typename T, int D>
+// grid (tile, kv-head, batch of K). HBM-bound: one read of K and V, by the first slab that is swept.
+constexpr uint8_t kUnseen = 2;  // a tile not looked at: no slab so far was swept
+template <typename T, int D, int GQ>
 __global__ __launch_bounds__(LSA_BLOCK) void tile_finite_kernel(RowsArgs a, uint8_t* odd) {
   constexpr int SEGS = D / 8, N = kTile * SEGS / LSA_BLOCK;
   __shared__ int bad[LSA_WAVES];
+  using V = SlabVerdict<D, GQ, LSA_BLOCK>;
+  __shared__ typename V::Red red;
   const int tile = blockIdx.x, g = blockIdx.y, b = blockIdx.z;
+  uint8_t* state = odd + ((int64_t)b * gridDim.y + g) * a.n_tile + tile;
+  if (a.u0 != 0 && *state != kUnseen) return;  // uniform
+  const V slab(a);
+  slab.add_up(red);
+  __syncthreads();
+  if (slab.verdict(a, red) != kSweep) {
+    if (threadIdx.x == 0) *state = kUnseen;
+    return;
+  }
   const T* kb = (const T*)a.k + b * a.kv_sb + g * a.kv_sh;
   const T* vb = (const T*)a.v + b * a.kv_sb + g * a.kv_sh;
   uint4 x[2 * N];
@@ -102,8 +180,7 @@ __global__ __launch_bounds__(LSA_BLOCK) void tile_finite_kernel(RowsArgs a, uint
   const uint64_t m = __ballot(o);
   if ((threadIdx.x & 63) == 0) bad[threadIdx.x / 64] = m != 0;
   __syncthreads();
-  if (threadIdx.x == 0)
-    odd[((int64_t)b * gridDim.y + g) * a.n_tile + tile] = (uint8_t)(bad[0] | bad[1] | bad[2] | bad[3]);
+  if (threadIdx.x == 0) *state = (uint8_t)(bad[0] | bad[1] | bad[2] | bad[3]);
 }
 
 // ---------------------------------------------------------------- bitmaps
@@ -114,7 +191,8 @@ constexpr int kSegWords = kSegKeys / 32 + 2;     // dwords of a row in LDS (two 
 
 struct BitLds {
   uint32_t w[kBlockRows][kSegWords];
-  int dup[kBlockRows];
+  int dup[kBlockRows], len[kBlockRows];
+  int tiles;
 };
 
 // One 32-row block (grid: row tile of the slab, kv-head when lists are per head, block). Two
@@ -129,7 +207,9 @@ __global__ __launch_bounds__(kBitThreads) void row_bits_kernel(RowsArgs a) {
   const int64_t u = a.u0 + (a.per_head ? x / a.Hkv : x);
   const int64_t b = u / a.n_rt;
   const int64_t t0 = ((u % a.n_rt) * a.rb + rb) * kBlockRows;
-  if (tid < kBlockRows) sh.dup[tid] = 0;
+  if (tid < kBlockRows) sh.dup[tid] = sh.len[tid] = 0;
+  if (tid == 0) sh.tiles = 0;
+  if (blk == 0 && tid < kXcds) a.left_n[tid] = 0;
   for (int64_t k0 = 0; k0 < a.Tk; k0 += kSegKeys) {
     for (int i = tid; i < kBlockRows * kSegWords; i += kBitThreads) (&sh.w[0][0])[i] = 0;
     __syncthreads();
@@ -141,6 +221,7 @@ __global__ __launch_bounds__(kBitThreads) void row_bits_kernel(RowsArgs a) {
         const int64_t li = list_of(a, b, t, g);
         int n = a.lengths[li];
         n = n < 0 ? 0 : (n > a.W ? a.W : n);
+        if (lane == 0) sh.len[r] = n;
         const int32_t* list = a.ids + li * a.W;
         bool twice = false;
         for (int j0 = 0; j0 < n; j0 += 8 * 64) {
@@ -166,16 +247,28 @@ __global__ __launch_bounds__(kBitThreads) void row_bits_kernel(RowsArgs a) {
     __syncthreads();
     const int tiles = (int)min((int64_t)kSegKeys / kTile, (a.Tk - k0 + kTile - 1) / kTile);
     const int tile0 = (int)(k0 / kTile);
+    int on = 0;
     for (int i = tid; i < tiles * kBlockRows; i += kBitThreads) {  // 64 lanes: two tiles of 32 rows
       const int tile = i / kBlockRows, r = i % kBlockRows;
       const uint64_t word = *(const uint64_t*)&sh.w[r][2 * tile];
       a.bits[(blk * a.n_tile + tile0 + tile) * kBlockRows + r] = word;
       const uint64_t m = __ballot(word != 0);
-      if (r == 0) a.any[blk * a.n_tile + tile0 + tile] = (uint8_t)(((lane ? m >> 32 : m) & 0xFFFFFFFFull) != 0);
+      if (r == 0) {
+        const int any = ((lane ? m >> 32 : m) & 0xFFFFFFFFull) != 0;
+        a.any[blk * a.n_tile + tile0 + tile] = (uint8_t)any;
+        on += any;
+      }
     }
+    on = wave_sum(on);
+    if (lane == 0) atomicAdd(&sh.tiles, on);
     __syncthreads();
   }
-  if (tid < kBlockRows) a.dup[blk * kBlockRows + tid] = (uint8_t)sh.dup[tid];
+  if (tid < LSA_WAVE) {
+    const bool dup = tid < kBlockRows && sh.dup[tid] != 0;
+    if (tid < kBlockRows) a.dup[blk * kBlockRows + tid] = (uint8_t)dup;
+    const int keys = wave_sum(tid < kBlockRows && !dup ? sh.len[tid] : 0);
+    if (tid == 0) a.listed[blk] = make_int2(keys, sh.tiles);
+  }
 }
 
 // ---------------------------------------------------------------- the sweep
@@ -200,17 +293,10 @@ struct alignas(1024) SweepLds {
   uint16_t v[NB][kTile * D];  // by vseg
   uint64_t mask[kWaves][NB][kBlockRows];
   uint16_t act[kMaxTiles];    // the tiles swept, ascending
-  int wsum[kWaves], wkeys[kWaves];
-  int bad, n_act;
+  int wsum[kWaves], wbad[kWaves];
+  typename SlabVerdict<D, 1, kThreads>::Red red;
+  int n_act, left0;
 };
-
-// Listed keys a swept tile under which the gather reads a workgroup's rows faster: the sweep
-// takes a CU ~2.6 us a tile (D 64: 1.9), the gather ~7.9 ns a listed key (D 64: 2.7, 3.8, 5.9
-// and 12.3 ns at query groups 1, 2, 4 and 8).
-template <int D, int GQ>
-__device__ constexpr int sparse_keys() {
-  return D == 128 ? 330 : (GQ == 1 ? 700 : (GQ == 2 ? 500 : (GQ == 4 ? 320 : 155)));
-}
 
 // Which LDS segment of row r holds its segment 0 (XOR): K rows are read 16 rows to a
 // 16-lane group at one segment, V rows (transposing reads) 8 rows at 64 bytes each.
@@ -533,17 +619,12 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 
   // the tiles any of the workgroup's rows lists, and whether one of them is not finite
   {
-    if (tid == 0) sh.bad = 0;
-    // the keys its rows list (shared or this kv-head's lists)
-    const int64_t tr = (u % a.n_rt) * RB * kBlockRows + tid;
-    int listed = 0;
-    if (tid < RB * kBlockRows && tr < a.Tq) {
-      const int len = a.lengths[list_of(a, b, tr, g)];
-      listed = len < 0 ? 0 : (len > a.W ? a.W : len);
-    }
-    listed = wave_sum(listed);
-    if (lane == 0) sh.wkeys[w] = listed;
-    __syncthreads();
+    const SlabVerdict<D, GQ, kThreads> slab(a);  // its loads and the next are in flight until the tiles are listed
+    int keys = 0;
+#pragma unroll
+    for (int r = 0; r < RB; ++r) keys += a.listed[blk0 + r].x;
+    const bool dup = tid < RB * kBlockRows && a.dup[blk0 * kBlockRows + tid];
+    bool not_finite = false;
     const uint8_t* odd = a.odd + ((a.kv_sb ? b : 0) * a.Hkv + g) * a.n_tile;
     int base = 0;
     for (int c0 = 0; c0 < a.n_tile; c0 += kThreads) {
@@ -553,7 +634,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
       for (int r = 0; r < RB; ++r) on |= a.any[(blk0 + r) * a.n_tile + tc];
       const bool use = tile < a.n_tile && on;
-      if (use && odd[tc]) sh.bad = 1;
+      not_finite |= use && odd[tc];
       const uint64_t m = __ballot(use);
       if (lane == 0) sh.wsum[w] = __popcll(m);
       __syncthreads();
@@ -567,17 +648,37 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
       base += total;
       __syncthreads();
     }
-    if (tid == 0) {
-      int keys = 0;
-      for (int x = 0; x < kWaves; ++x) keys += sh.wkeys[x];
-      if (keys < base * sparse_keys<D, GQ>()) sh.bad = 1;
-      sh.n_act = base;
-      a.rest[(int64_t)ul * a.Hkv + g] = (uint8_t)sh.bad;
-    }
+    slab.add_up(sh.red);
+    const bool wave_bad = __any(not_finite);
+    if (lane == 0) sh.wbad[w] = wave_bad;
     __syncthreads();
+    bool bad = false;
+#pragma unroll
+    for (int x = 0; x < kWaves; ++x) bad |= sh.wbad[x] != 0;
+    const bool all = bad || keys < base * sparse_keys<D, GQ>() || slab.verdict(a, sh.red) == kGather;  // uniform
+    if (tid == 0) sh.n_act = all ? -1 : base;
+    // the rows the gather reads: all, or the ones that list a key twice
+    const int64_t tr = (u % a.n_rt) * RB * kBlockRows + tid;
+    const bool left = tid < RB * kBlockRows && tr < a.Tq && (all || dup);
+    const uint64_t m = __ballot(left);
+    if (lane == 0) sh.wsum[w] = __popcll(m);
+    __syncthreads();
+    int before = 0, total = 0;
+#pragma unroll
+    for (int x = 0; x < kWaves; ++x) {
+      before += x < w ? sh.wsum[x] : 0;
+      total += sh.wsum[x];
+    }
+    if (total > 0) {  // uniform
+      const int c = (int)(((int64_t)ul * a.Hkv + g) % kXcds);
+      if (tid == 0) sh.left0 = atomicAdd(&a.left_n[c], total);
+      __syncthreads();
+      const int at = sh.left0 + before + __popcll(m & ((1ull << lane) - 1));
+      if (left) a.left[(int64_t)c * a.left_cap + at] = (int32_t)(((int64_t)ul * RB * kBlockRows + tid) * a.Hkv + g);
+    }
   }
-  if (sh.bad) return;  // uniform
   const int n = __builtin_amdgcn_readfirstlane(sh.n_act);
+  if (n < 0) return;  // uniform
 
   const bool row_ok = t < a.Tq;
   const int64_t qrow = ((b * a.Tq + (row_ok ? t : 0)) * a.Hq + (int64_t)g * GQ + hl) * D;
@@ -682,55 +783,64 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 
 // ---------------------------------------------------------------- the rows left to the gather
 
-// Every workgroup looks at 256 (row, kv-head) units at a time and reads the ones left out.
+// The units (row, kv-head) the sweep left, from their lists, so that wherever they lie they spread over
+// the chip; up to kRestGrid of them a workgroup each, as their lengths may differ. The rows of a
+// (row tile, kv-head), which list much the same, are in one list, and a list goes to the workgroups of one
+// XCD (consecutive ones are on different XCDs), whose L2 then serves them all; where the lists
+// differ much in length, the workgroups take them one after the other instead. All units left, 32
+// heads on 8, D 128 (us; a workgroup of the gather alone for each unit / this call, with the bitmaps and a sweep
+// that finds nothing to do / before, when a workgroup read all it found in 256 neighbouring
+// units): 1024 rows of 1024 keys, one twice 301 / 329 / 3550, of 16 keys of 1024 60 / 79 / 900; 2048
+// rows of 0 to 4612 keys of 32768 1400 / 1465 / 8970. Taking units one by one from a counter costs
+// ~26 ns each across the XCDs (1024 rows of 16 keys: 650 us). 2048 workgroups: the last figure is
+// 1800, but with nothing left they are 1.5 us less.
 template <typename T, int D, int GQ>
-__global__ __launch_bounds__(LSA_BLOCK) void rows_rest_kernel(RowsArgs a) {
+__global__ __launch_bounds__(LSA_BLOCK) __attribute__((amdgpu_waves_per_eu(GQ == 8 ? 2 : 3))) void rows_rest_kernel(
+    RowsArgs a) {
   using S = ReadShape<T, D, GQ>;
-  constexpr int RB = kWaves / GQ, RT = RB * kBlockRows;
+  constexpr int RT = kWaves / GQ * kBlockRows;
   __shared__ ReadLds<D, GQ, kMaxSplits> sh;
-  __shared__ uint64_t todo[LSA_WAVES];
-  const int tid = threadIdx.x;
-  const int lp = (tid & 63) % S::LPT;
-  const int64_t units = (int64_t)a.n_u * RT * a.Hkv;  // row tile, row, kv-head
-  for (int64_t base = (int64_t)blockIdx.x * LSA_BLOCK; base < units; base += (int64_t)gridDim.x * LSA_BLOCK) {
-    const int64_t i = base + tid;
-    bool left = false;
-    if (i < units) {
-      const int g = (int)(i % a.Hkv);
-      const int64_t x = i / a.Hkv, ul = x / RT;
-      const int r = (int)(x % RT);
-      const int64_t blk = (a.per_head ? ul * a.Hkv + g : ul) * RB + r / kBlockRows;
-      left = a.rest[ul * a.Hkv + g] || a.dup[blk * kBlockRows + r % kBlockRows];
-      left &= ((a.u0 + ul) % a.n_rt) * RT + r < a.Tq;
+  const int lp = (threadIdx.x & 63) % S::LPT;
+  int most = 0, total = 0;
+#pragma unroll
+  for (int c = 0; c < kXcds; ++c) {
+    most = max(most, a.left_n[c]);
+    total += a.left_n[c];
+  }
+  const bool even = most <= 2 * (total / kXcds);
+  const int end = even ? most * kXcds : total;
+  for (int i = blockIdx.x; i < end; i += gridDim.x) {  // uniform
+    int c = even ? i % kXcds : 0, p = even ? i / kXcds : i;
+    if (even) {
+      if (p >= a.left_n[c]) continue;
+    } else {
+      while (p >= a.left_n[c]) p -= a.left_n[c++];
     }
-    const uint64_t m = __ballot(left);
-    if ((tid & 63) == 0) todo[tid / 64] = m;
-    __syncthreads();
-    for (int wv = 0; wv < LSA_WAVES; ++wv) {
-      for (uint64_t left_m = todo[wv]; left_m; left_m &= left_m - 1) {  // uniform
-        const int64_t j = base + 64 * wv + (__ffsll((long long)left_m) - 1);
-        const int g = (int)(j % a.Hkv);
-        const int64_t x = j / a.Hkv, u = a.u0 + x / RT;
-        const int64_t b = u / a.n_rt, t = (u % a.n_rt) * RT + x % RT;
-        const int64_t li = list_of(a, b, t, g);
-        int n = a.lengths[li];
-        n = n < 0 ? 0 : (n > a.W ? a.W : n);
-        const int32_t* list = a.ids + li * a.W;
-        const T* kb = (const T*)a.k + b * a.kv_sb + g * a.kv_sh + lp * S::VEC;
-        const T* vb = (const T*)a.v + b * a.kv_sb + g * a.kv_sh + lp * S::VEC;
-        const int64_t qo = ((b * a.Tq + t) * a.Hq + (int64_t)g * GQ) * D;
-        AttnState<T, D, GQ> st;
-        attend_span<T, D, GQ>((const T*)a.q + qo, kb, vb, a.kv_st, a.Tk, 0, n,
-                              [&](int s) {
-                                const int32_t id = n > 0 ? list[s < n ? s : n - 1] : -1;
-                                return s < n ? id : -1;
-                              },
-                              a.scale_log2, st);
-        finish_span<T, D, GQ, kMaxSplits, true>(sh, st, true, (T*)a.out + qo, nullptr, a.empty_nan);
-        __syncthreads();  // sh is used again
-      }
+    const uint32_t j = (uint32_t)__builtin_amdgcn_readfirstlane(a.left[(int64_t)c * a.left_cap + p]);
+    const int g = (int)(j % (uint32_t)a.Hkv);
+    const uint32_t x = j / (uint32_t)a.Hkv;
+    const int64_t u = a.u0 + x / RT;
+    const int64_t b = u / a.n_rt, t = (u % a.n_rt) * RT + x % RT;
+    const int64_t li = list_of(a, b, t, g);
+    int n = a.lengths[li];
+    n = n < 0 ? 0 : (n > a.W ? a.W : n);
+    T* outp = (T*)a.out + ((b * a.Tq + t) * a.Hq + (int64_t)g * GQ) * D;
+    if (n == 0) {
+      for (int o = threadIdx.x; o < GQ * D; o += LSA_BLOCK) store_out<T>(outp + o, a.empty_nan ? NAN : 0.0f);
+      continue;
     }
-    __syncthreads();
+    const int32_t* list = a.ids + li * a.W;
+    const T* kb = (const T*)a.k + b * a.kv_sb + g * a.kv_sh + lp * S::VEC;
+    const T* vb = (const T*)a.v + b * a.kv_sb + g * a.kv_sh + lp * S::VEC;
+    AttnState<T, D, GQ> st;
+    attend_span<T, D, GQ>((const T*)a.q + (outp - (T*)a.out), kb, vb, a.kv_st, a.Tk, 0, n,
+                          [&](int s) {
+                            const int32_t id = list[s < n ? s : n - 1];
+                            return s < n ? id : -1;
+                          },
+                          a.scale_log2, st);
+    __syncthreads();  // the last unit is done with sh
+    finish_span<T, D, GQ, kMaxSplits, true>(sh, st, true, outp, nullptr, a.empty_nan);
   }
 }
 
@@ -739,7 +849,8 @@ __global__ __launch_bounds__(LSA_BLOCK) void rows_rest_kernel(RowsArgs a) {
 struct Layout {
   int gq, rb;
   int64_t n_rt, n_tile, u_total, slab_u, blocks;
-  size_t bits, any, dup, rest, odd, total;
+  int64_t left_cap;
+  size_t bits, any, dup, listed, left_n, left, odd, total;
 };
 
 Layout layout_of(int64_t B, int64_t Tq, int64_t Tk, int32_t Hq, int32_t Hkv, int per_head) {
@@ -750,40 +861,45 @@ Layout layout_of(int64_t B, int64_t Tq, int64_t Tk, int32_t Hq, int32_t Hkv, int
   l.n_tile = (Tk + kTile - 1) / kTile;
   l.u_total = B * l.n_rt;
   const int64_t per_u = (int64_t)l.rb * (per_head ? Hkv : 1);  // blocks a row tile
-  const int64_t fit = kSlabBytes / (per_u * l.n_tile * kBlockRows * 8);
+  const int64_t units_u = (int64_t)l.rb * kBlockRows * Hkv;     // (row, kv-head) units a row tile
+  const int64_t most = per_u * l.n_tile * kBlockRows * 8;       // bytes of bitmaps a row tile
+  const int64_t fit = kSlabBytes / (most > units_u * 4 ? most : units_u * 4);
   l.slab_u = fit < 1 ? 1 : (fit < l.u_total ? fit : l.u_total);
   l.blocks = l.slab_u * per_u;
   auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };
   l.bits = 0;
   l.any = l.bits + up((size_t)l.blocks * l.n_tile * kBlockRows * 8);
   l.dup = l.any + up((size_t)l.blocks * l.n_tile);
-  l.rest = l.dup + up((size_t)l.blocks * kBlockRows);
-  l.odd = l.rest + up((size_t)l.slab_u * Hkv);
+  l.listed = l.dup + up((size_t)l.blocks * kBlockRows);
+  l.left_n = l.listed + up((size_t)l.blocks * sizeof(int2));
+  l.left = l.left_n + up(kXcds * sizeof(int));
+  l.left_cap = (l.slab_u * Hkv + kXcds - 1) / kXcds * l.rb * kBlockRows;
+  l.odd = l.left + up((size_t)(kXcds * l.left_cap) * sizeof(int32_t));
   l.total = l.odd + up((size_t)B * Hkv * l.n_tile);
   return l;
 }
 
 template <typename T, int D, int GQ>
-void launch_slab(const RowsArgs& a, const Layout& l, hipStream_t s) {
+void launch_slab(const RowsArgs& a, const Layout& l, int64_t kv_batches, uint8_t* odd, hipStream_t s) {
   const int64_t per_u = (int64_t)l.rb * (a.per_head ? a.Hkv : 1);
   row_bits_kernel<<<dim3((unsigned)(a.n_u * per_u)), kBitThreads, 0, s>>>(a);
+  const dim3 tiles((unsigned)l.n_tile, (unsigned)a.Hkv, (unsigned)kv_batches);
+  tile_finite_kernel<T, D, GQ><<<tiles, LSA_BLOCK, 0, s>>>(a, odd);
   rows_mfma_kernel<T, D, GQ><<<dim3((unsigned)(a.n_u * a.Hkv)), kThreads, 0, s>>>(a);
   const int64_t units = (int64_t)a.n_u * l.rb * kBlockRows * a.Hkv;
-  const int64_t blocks = (units + LSA_BLOCK - 1) / LSA_BLOCK;
-  rows_rest_kernel<T, D, GQ><<<dim3((unsigned)(blocks < 2048 ? blocks : 2048)), LSA_BLOCK, 0, s>>>(a);
+  rows_rest_kernel<T, D, GQ><<<dim3((unsigned)(units < kRestGrid ? units : kRestGrid)), LSA_BLOCK, 0, s>>>(a);
 }
 
 template <typename T, int D>
 void launch_rows(RowsArgs a, const Layout& l, int64_t kv_batches, uint8_t* odd, hipStream_t s) {
-  tile_finite_kernel<T, D><<<dim3((unsigned)l.n_tile, (unsigned)a.Hkv, (unsigned)kv_batches), LSA_BLOCK, 0, s>>>(a, odd);
   for (int64_t u = 0; u < l.u_total; u += l.slab_u) {
     a.u0 = u;
     a.n_u = (int)(l.u_total - u < l.slab_u ? l.u_total - u : l.slab_u);
     switch (l.gq) {
-      case 1: launch_slab<T, D, 1>(a, l, s); break;
-      case 2: launch_slab<T, D, 2>(a, l, s); break;
-      case 4: launch_slab<T, D, 4>(a, l, s); break;
-      default: launch_slab<T, D, 8>(a, l, s); break;
+      case 1: launch_slab<T, D, 1>(a, l, kv_batches, odd, s); break;
+      case 2: launch_slab<T, D, 2>(a, l, kv_batches, odd, s); break;
+      case 4: launch_slab<T, D, 4>(a, l, kv_batches, odd, s); break;
+      default: launch_slab<T, D, 8>(a, l, kv_batches, odd, s); break;
     }
   }
 }
@@ -821,7 +937,8 @@ extern "C" int lsa_read_rows(const void* q, const void* k, const void* v, int dt
   const Layout l = layout_of(B, Tq, Tk, Hq, Hkv, ids_per_head ? 1 : 0);
   LSA_REQUIRE(scratch && ((uintptr_t)scratch & 255) == 0 && scratch_bytes >= l.total, LSA_ERR_WORKSPACE,
               "lsa_read_rows: scratch %zu < %zu bytes", scratch_bytes, l.total);
-  LSA_REQUIRE(l.blocks <= 0x7FFFFFFF && l.slab_u * Hkv <= 0x7FFFFFFF, LSA_ERR_SHAPE, "lsa_read_rows: too many rows");
+  LSA_REQUIRE(l.blocks <= 0x7FFFFFFF && l.slab_u * l.rb * kBlockRows * Hkv <= 0x7FFFFFFF, LSA_ERR_SHAPE,
+              "lsa_read_rows: too many rows");
   RowsArgs a;
   char* ws = (char*)scratch;
   a.q = q; a.k = k; a.v = v; a.out = out; a.ids = ids; a.lengths = lengths;
@@ -829,7 +946,8 @@ extern "C" int lsa_read_rows(const void* q, const void* k, const void* v, int dt
   a.Hq = Hq; a.Hkv = Hkv; a.W = W; a.per_head = ids_per_head ? 1 : 0;
   a.u0 = 0; a.n_u = 0; a.n_rt = (int)l.n_rt; a.rb = l.rb; a.n_tile = (int)l.n_tile;
   a.bits = (uint64_t*)(ws + l.bits); a.any = (uint8_t*)(ws + l.any); a.dup = (uint8_t*)(ws + l.dup);
-  a.rest = (uint8_t*)(ws + l.rest); a.odd = (const uint8_t*)(ws + l.odd);
+  a.listed = (int2*)(ws + l.listed); a.left_n = (int*)(ws + l.left_n); a.left = (int32_t*)(ws + l.left);
+  a.left_cap = (int)l.left_cap; a.odd = (const uint8_t*)(ws + l.odd);
   a.scale_log2 = scale * kLog2e; a.empty_nan = empty_nan ? 1 : 0;
   const int64_t kv_batches = kv_batch_stride ? B : 1;
   uint8_t* odd = (uint8_t*)(ws + l.odd);
