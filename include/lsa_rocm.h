@@ -249,8 +249,9 @@ int lsa_read(const void* q, const void* k, const void* v, int dtype, int64_t B, 
  * row's list a bitmap that masks its weights (two 16-bit halves that add up to the fp32 weight
  * within 2^-17 of it in bf16, and in fp16 within 2^-23 of it or 2^-37 of the row's largest weight,
  * whichever is more). Rows the sweep does not serve - a list naming a key twice, a tile whose K or V
- * is not finite, too few listed keys for the tiles crossed - are read by the gather in the
- * same call. Arguments as lsa_read's; bf16/fp16 rows of head dim 64 or 128, at most 262144
+ * is not finite, too few listed keys for the tiles crossed (of 256 columns, or of most of the
+ * call) - are read by the gather in the same call. Within either read a row's bits do not depend on the
+ * other rows. Arguments as lsa_read's; bf16/fp16 rows of head dim 64 or 128, at most 262144
  * cache rows, kv_token_stride below 2^24, scale > 0. lsa_read_rows_scratch_bytes(): 0 where it
  * does not apply; scratch 256-byte aligned, no initialisation. */
 size_t lsa_read_rows_scratch_bytes(int dtype, int64_t B, int64_t Tq, int64_t Tk, int32_t Hq, int32_t Hkv, int32_t D,

@@ -6,7 +6,9 @@ shares each gathered K/V row, fetched once as 16-byte coalesced loads; scores an
 the online softmax are fp32; when there are few rows (decode) each list is split
 over several workgroups and the last one to finish merges their softmax partials. Many rows
 over one cache (a prefill's) go to a masked sweep on the matrix cores instead where that is
-faster (``_sweep_pays``).
+faster (``_sweep_pays``). The two round differently, and which of them reads a row depends on the
+call's sizes and on how many keys its neighbours list and whether the tiles they list are
+finite; within either, a row's bits do not depend on the other rows.
 Contract as the reference: -1 ids and slots past a row's length are skipped,
 duplicates count per occurrence, a row with no keys gives zeros, the output has q's
 dtype. Lists are [B, Tq, W] shared by all heads or [B, Tq, Hkv, W] per kv-head

@@ -207,6 +207,23 @@ def test_large_scores():
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("D", [64, 128])
+def test_a_swept_row_does_not_depend_on_its_neighbours(dtype, D):
+    """The same rows beside others whose scores are 30 times as large and whose lists are other
+    keys: bit for bit the same."""
+    q, k, v, ids, lengths = make(dtype, 1, 64, 1024, 8, 2, D, 1024, seed=11)
+    ids[:] = torch.stack([torch.randperm(1024, generator=torch.Generator().manual_seed(t)) for t in range(64)])
+    lengths[:] = 700
+    alone = sweep(q, k, v, ids, lengths)
+    q[:, 1::2] *= 30
+    ids[:, 1::2] = ids[:, 1::2].flip(-1)
+    other = sweep(q, k, v, ids, lengths)
+    torch.cuda.synchronize()
+    assert torch.equal(alone[:, ::2], other[:, ::2])
+    assert not torch.equal(alone[:, 1::2], other[:, 1::2])
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("n", [4611, 40000])
 def test_small_weights_beside_a_large_one(dtype, n):
     """A row of one key of weight 1 (V 0) and n of weight 2^-x (V 1): what is read is the small
