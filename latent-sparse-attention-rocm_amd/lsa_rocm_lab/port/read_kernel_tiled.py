@@ -62,6 +62,8 @@ def _sweep_pays(dtype, B: int, Tq: int, Tk: int, Hq: int, Hkv: int, D: int, widt
     Hkv 1, D 64 37 / 106 us at 2048, 346 / 311 at 8192."""
     if dtype not in (torch.bfloat16, torch.float16) or D not in _TILE_US or not 0.0 < scale < math.inf:
         return False
+    if os.environ.get("LSA_READ_SPLITS"):  # a split count is asked for: the gather's
+        return False
     group = Hq // Hkv
     if group not in _GATHER_64 or token_stride >= 1 << 24 or Tk < 1 or width < 1:
         return False
