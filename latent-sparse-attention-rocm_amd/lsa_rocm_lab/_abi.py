@@ -218,7 +218,8 @@ class Workspace:
     """Scratch per (device, stream, purpose), grown on demand; kernels fully write the
     part they read, so it needs no initialisation. Calls sharing it are stream-ordered.
     A buffer that is outgrown is retired, never freed: a HIP graph captured earlier may
-    still replay against it."""
+    still replay against it. So a buffer at least doubles when it grows: sizes that creep up
+    (prompts of ever more rows) retire less than one more buffer in all, not one a size."""
 
     _buffers: dict[tuple, torch.Tensor] = {}
     _retired: list[torch.Tensor] = []
@@ -232,6 +233,7 @@ class Workspace:
         if buf is None or buf.numel() < nbytes:
             if buf is not None:
                 cls._retired.append(buf)
+                nbytes = max(nbytes, 2 * buf.numel())
             buf = torch.empty(max(nbytes, 1 << 16), dtype=torch.uint8, device=device)
             cls._buffers[key] = buf
         return buf
