@@ -188,9 +188,16 @@ def ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
+# torch's own query of a stream's handle; not part of its public interface
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream(device: torch.device | None = None) -> int:
-    """The current stream's handle (without making a ``torch.cuda.Stream`` of it)."""
-    return torch._C._cuda_getCurrentRawStream(device_index(device))
+    """The current stream's handle (without making a ``torch.cuda.Stream`` of it where this
+    torch can tell the handle alone)."""
+    if _raw_stream is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return _raw_stream(device_index(device))
 
 
 def device_index(device: torch.device | int | str | None) -> int:

@@ -291,3 +291,14 @@ def test_workspaces_of_creeping_sizes_stay_bounded(monkeypatch):
     held = buf.numel() + sum(b.numel() for b in _abi.Workspace._retired)
     assert held < 4 * 200 * step
     assert _abi.Workspace.get(cpu, "test", 0) is None
+
+
+def test_stream_without_torchs_private_query(monkeypatch):
+    class Stream:
+        cuda_stream = 1234
+
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: Stream())
+    monkeypatch.setattr(_abi, "_raw_stream", None)
+    assert _abi.stream(torch.device("cuda", 0)) == 1234
+    monkeypatch.setattr(_abi, "_raw_stream", lambda index: 100 + index)
+    assert _abi.stream(torch.device("cuda", 3)) == 103
