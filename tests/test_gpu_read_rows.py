@@ -17,7 +17,8 @@ import torch
 
 import oracle
 from lsa_rocm_lab import _abi
-from lsa_rocm_lab.port.read_kernel_tiled import _sparse_read
+from lsa_rocm_lab.port import pipeline
+from lsa_rocm_lab.port.read_kernel_tiled import _sparse_read, _sweep_pays
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -264,3 +265,104 @@ def test_segments_and_slabs():
     lengths = torch.full((B, Tq), W, dtype=torch.int32)
     rows = [0, 31, 32, 1000, 2047, 2048, 2079]
     check(q, k, v, ids, lengths, rows=rows)
+
+
+def _views(kind, B, Tk, Hkv, D, dtype, g):
+    """K and V as a program may hold them: strides of a longer cache, of heads before tokens, of a
+    fused projection's rows, of one pool."""
+    draw = lambda *shape: torch.randn(*shape, device=DEV, generator=g).to(dtype)
+    if kind == "longer":  # the first Tk rows of a cache
+        return draw(B, Tk + 300, Hkv, D)[:, :Tk], draw(B, Tk + 300, Hkv, D)[:, :Tk]
+    if kind == "heads first":
+        return draw(B, Hkv, Tk, D).transpose(1, 2), draw(B, Hkv, Tk, D).transpose(1, 2)
+    if kind == "fused":  # q, k and v of a token side by side
+        rows = draw(B, Tk, 6 * Hkv, D)
+        return rows[:, :, 4 * Hkv:5 * Hkv], rows[:, :, 5 * Hkv:]
+    assert kind == "pool"
+    return draw(1, Tk, Hkv, D), draw(1, Tk, Hkv, D)
+
+
+@pytest.mark.parametrize("per_head", [False, True])
+@pytest.mark.parametrize("kind,dtype", [("longer", torch.bfloat16), ("heads first", torch.float16),
+                                        ("fused", torch.bfloat16), ("pool", torch.float16)])
+def test_public_reads_of_cache_views(monkeypatch, kind, dtype, per_head):
+    """``lsa_read`` over views of a cache: read in place by the sweep, against the gather."""
+    B, Tq, Tk, Hq, Hkv, D, W = 2, 768, 1000, 32, 8, 128, 1000
+    g = torch.Generator(device=DEV).manual_seed(13)
+    q = torch.randn(B, Tq, Hq, D, device=DEV, generator=g).to(dtype)
+    k, v = _views(kind, B, Tk, Hkv, D, dtype, g)
+    lead = (B, Tq, Hkv) if per_head else (B, Tq)
+    ids = torch.rand(*lead, W, device=DEV, generator=g).argsort(-1).to(torch.int32)
+    lengths = torch.randint(500, W + 1, lead, device=DEV, generator=g).to(torch.int32)
+    called, call = [], _abi.call
+    monkeypatch.setattr(_abi, "call", lambda name, *a: (called.append((name, a)), call(name, *a))[1])
+    got = pipeline.lsa_read(q, k, v, ids, lengths, D ** -0.5)
+    name, args = called[0]
+    assert name == "lsa_read_rows" and args[1] == k.data_ptr()  # no copy
+    want = _sparse_read(q, k, v, ids, lengths, None, False, splits=1)
+    assert called[1][0] == "lsa_read"
+    torch.cuda.synchronize()
+    err, ref = (got.float() - want.float()).abs(), want.float().abs()
+    # the two reads' own rounding, and the weights and scores of both
+    assert (err <= 2 * RTOL[dtype] * ref + 2.0 ** -12 * v.abs().max().item()).all(), err.max()
+
+
+def test_the_widest_token_stride():
+    """Tokens 2^24 - 8 elements apart, the widest the sweep takes: 63 rows of a tile are 2 GB."""
+    D, Tk, stride = 64, 130, (1 << 24) - 8
+    g = torch.Generator(device=DEV).manual_seed(14)
+    store = torch.empty((Tk - 1) * stride + 2 * D, device=DEV, dtype=torch.bfloat16)
+    k, v = (torch.as_strided(store, (1, Tk, 1, D), (0, stride, D, 1), off) for off in (0, D))
+    for t in (k, v):
+        t.copy_(torch.randn(1, Tk, 1, D, device=DEV, generator=g))
+    q = torch.randn(1, 64, 4, D, device=DEV, generator=g).to(torch.bfloat16)
+    ids = torch.rand(1, 64, Tk, device=DEV, generator=g).argsort(-1).to(torch.int32)
+    lengths = torch.full((1, 64), Tk, device=DEV, dtype=torch.int32)
+    nbytes = _abi.size("lsa_read_rows_scratch_bytes", _abi.LSA_BF16, 1, 64, Tk, 4, 1, D, Tk, 0)
+    ws, out = torch.empty(nbytes, dtype=torch.uint8, device=DEV), torch.empty_like(q)
+    print(f"rows sweep token stride {stride}", flush=True)
+    _abi.call("lsa_read_rows", q.data_ptr(), k.data_ptr(), v.data_ptr(), _abi.LSA_BF16, 1, 64, Tk, 4, 1, D, 0, stride, D,
+              ids.data_ptr(), lengths.data_ptr(), Tk, 0, D ** -0.5, 0, ws.data_ptr(), nbytes, out.data_ptr(),
+              _abi.stream(out.device))
+    dense = sweep(*(t.cpu() for t in (q, k, v, ids, lengths)))
+    torch.cuda.synchronize()
+    assert torch.equal(out, dense)
+
+
+def test_the_sweep_in_a_captured_graph():
+    """A read that goes to the sweep as a replayed graph, over new queries, lists and caches, some rows
+    left to the gather, with eager work between the replays."""
+    Tq, Hq, Hkv, D, W = 1024, 32, 8, 128, 1024
+    g = torch.Generator(device=DEV).manual_seed(15)
+    q, k, v = (torch.randn(1, Tq, h, D, device=DEV, generator=g).to(torch.bfloat16) for h in (Hq, Hkv, Hkv))
+    assert _sweep_pays(q.dtype, 1, Tq, Tq, Hq, Hkv, D, W, k.stride(1), D ** -0.5)
+    ids = torch.empty(1, Tq, W, device=DEV, dtype=torch.int32)
+    lengths = torch.empty(1, Tq, device=DEV, dtype=torch.int32)
+
+    def inputs():
+        for t in (q, k, v):
+            t.copy_(torch.randn(t.shape, device=DEV, generator=g))
+        ids.copy_(torch.rand(ids.shape, device=DEV, generator=g).argsort(-1))
+        ids[:, ::9, 0] = ids[:, ::9, 1]  # for the gather
+        lengths.copy_(torch.randint(300, W + 1, lengths.shape, device=DEV, generator=g))
+
+    def step():
+        return pipeline.lsa_read(q, k, v, ids, lengths, D ** -0.5)
+
+    inputs()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step()
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        out = step()
+    for _ in range(4):
+        inputs()
+        want = step().clone()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)

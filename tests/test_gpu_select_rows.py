@@ -116,7 +116,8 @@ def test_default_chain_equals_the_listing(monkeypatch, G, rows, top_p):
 
 
 def test_rows_select_and_read_in_a_captured_graph():
-    """The many-row select and read as a replayed graph, over new inputs, with eager work between."""
+    """The many-row select, and a read of its lists (by the gather at this size), as a replayed graph, over
+    new inputs, with eager work between."""
     gen = torch.Generator(device=DEV).manual_seed(9)
     R, rows, Hq, Hkv, D = 2048, 300, 8, 2, 64
     table, config = _table(0, rows, D, gen, False), _config(64)
@@ -148,3 +149,26 @@ def test_rows_select_and_read_in_a_captured_graph():
         torch.cuda.synchronize()
         for got, w in zip(out, want):
             assert torch.equal(got, w)
+
+
+@pytest.mark.parametrize("G", [0, 2])
+@pytest.mark.parametrize("spans", [False, True])
+def test_rows_select_of_a_paged_cache(monkeypatch, G, spans):
+    """Listed ids through a slot table, every query row by its own table row, some ids past the
+    table's width: as the general select maps them."""
+    gen = torch.Generator(device=DEV).manual_seed(21 + G)
+    R, rows, D = 311, 700, 64
+    table = _table(G, rows, D, gen, False, spans)
+    q = torch.randn(*((R, G) if G else (R,)), D, device=DEV, generator=gen)
+    pos = torch.randint(-1, 5 * rows, (R,), device=DEV, generator=gen).to(torch.int32)
+    slots = torch.stack([torch.randperm(4000, device=DEV, generator=gen)[:2500] for _ in range(5)]).to(torch.int32)
+    slots[:, ::50] = -1  # pages not there
+    which = torch.randint(0, 5, (R,), device=DEV, generator=gen).to(torch.int32)
+    config, got, called, call = _config(64), [], [], pipeline._abi.call
+    monkeypatch.setattr(pipeline._abi, "call", lambda name, *a: (called.append(name), call(name, *a))[1])
+    for tiles in (True, False):
+        monkeypatch.setattr(pipeline, "_rows_pay", lambda *a, tiles=tiles: tiles)
+        got.append(pipeline._fused_select(q, pos, table, config, config.top_k, "bf16", slots, which))
+    torch.cuda.synchronize()
+    assert called == ["lsa_select_rows", "lsa_select_flat"]
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
