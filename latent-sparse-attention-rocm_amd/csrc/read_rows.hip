@@ -280,11 +280,12 @@ __global__ __launch_bounds__(kBitThreads) void row_bits_kernel(RowsArgs a) {
 // apart (phase_barrier twice a step), so one group's matrix work runs beside the other's vector
 // work instead of all waves wanting the same unit at once.
 //
-// What bounds it (cycle counts of a wave, D 128): M ~2350 cycles against 1536 of matrix work
-// (issuing the five loads costs ~130 each, wherever they stand), V ~2600 (~330 vector
-// instructions, 32 of them exponentials, beside the other group's matrix instructions). 32k rows
-// of the reference's lists (4288 keys a row on average), Hq 32, Hkv 8, D 128: 10.8 ms against
-// 46.2 for the gather, 1220 TFLOP/s on the products of every swept pair with both halves.
+// What bounds it (counters, 32k rows of the reference's lists, 4288 keys a row on average, Hq 32,
+// Hkv 8, D 128): a step of both groups takes ~5530 cycles of a SIMD against 3072 of matrix work.
+// Matrix cores busy 55% of the cycles, vector unit 48% (~330 instructions a wave's V, 32 of them
+// exponentials), both at once 17%; waves wait 18%, no LDS bank conflicts; the five loads of an M
+// cost issue time wherever they stand. 10.7 ms against 46.2 for the gather; 403 M matrix
+// instructions, 13.2 TFLOP with both halves of every swept pair: 1235 TFLOP/s.
 
 
 template <int D>

@@ -5,10 +5,12 @@ a HIP kernel in liblsa_rocm.so:
 
 * ``visible_counts`` (pipeline.py:184-186), ``_production_scores`` (:217-232),
   ``best_first_keys`` (:189-214), ``flat_select_reference`` (:248-271) - the unfused
-  chain: score kernel -> listing pack -> radix top-k -> unpack -> expansion walk;
+  chain: visible counts -> scores -> radix top-k of the packed scores -> expansion walk from the
+  keys (past 4096 picks with the listing and the unpacked ids between);
 * ``flat_select`` (:274-316) with the ``LSA_SELECT_IMPL`` switch: ``fused`` is ONE
   kernel from the index queries to the read lists (score + top-k + expansion, split
-  over workgroups when there are few rows); ``fused_unpack`` keeps the listing +
+  over workgroups when there are few rows; many rows against one table a group take two,
+  the scores first); ``fused_unpack`` keeps the listing +
   top-k and expands from the keys; ``reference`` is the unfused chain;
 * ``tree_select`` (:319-337) over a one- to four-level hierarchy from
   ``build_hierarchy_gpu`` (:153-178), ``lsa_read`` (:373-375), ``position_buckets``
